@@ -130,8 +130,10 @@ typedef struct mvr_paged_attention_args {
 } mvr_paged_attention_args;
 
 /* Bytes of workspace mvr_paged_attention needs for these arguments (depends
-   only on the scalar fields; 0 when no sequence is split into context
-   partitions and page_size is a multiple of 16).  The workspace holds fp32
+   on the scalar fields and the planning hints; 0 when no sequence is split
+   into context partitions and page_size is a multiple of 16).  Only the key
+   splits of a prefill launch can do with less: such a call splits its keys as
+   far as the workspace it is given allows, down to not at all.  The workspace holds fp32
    partial results of the partitions and, when page_size is not a multiple of
    16, a copy of the batch's K/V in 16-token pages (num_seqs x
    ceil(max_seq_len / 16) pages) with its block table; its contents need no

@@ -11,6 +11,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <vector>
@@ -177,8 +178,114 @@ int device_cus() {
 struct LiveSeqs {
   int64_t count = 0;   // sequences with rows in this launch (0: num_seqs)
   int max_seq_len = 0; // their longest context (0: the call's max_seq_len)
-  int64_t split_count = 0; // prefill kernel: sequences given key splits and partial slots (0: num_seqs)
+  // Prefill kernel: valid host tables of the call, whose sequences of at least
+  // q_min new tokens are the launch's (null: count sequences at the bounds).
+  const int32_t* cu_q_lens = nullptr;
+  const int32_t* seq_lens = nullptr;
+  int q_min = 1;
+  // Largest workspace the balanced prefill grid's partials may take.
+  size_t prefill_budget = (size_t)48 << 20;
 };
+
+// Keys of one step of a prefill block: one key tile of 64 tokens (F32: 32)
+// per wavefront group, two groups up to D=128.
+int prefill_step_keys(const mvr_paged_attention_args* a) {
+  return (a->dtype == MVR_DTYPE_F16 ? 64 : 32) * (a->head_dim > 128 ? 1 : 2);
+}
+
+// Balanced prefill grid (each row tile's keys in parts of at most part_steps
+// steps, a block per part, and a merge launch) where the unsplit one, a block
+// per row tile, leaves CUs idle or waits for its longest sequence.
+// For one to four rounds of blocks over the CUs, and for fewer parts that leave
+// CUs idle: the shortest parts whose blocks fit, and their estimated time.
+// Measured at D=128 (one box, HIP events): a step of the two-group block takes
+// 1.5 us in F16 and 6.9 us in F32 alone and 0.5 / 0.9 us more with every CU
+// busy; a block costs 8 us beside its steps; a split call 5 us for the merge
+// and 11 us per CU-full of parts for their partial rows (64 KiB each, written
+// and read) and their cold start.  F16, 256 tokens on 2,048, 64 tiles: 37.0 us
+// unsplit, 36.1 / 33.7 / 36.0 in 2 / 3 / 4 parts; 64 on 8,128, 16 tiles: 102.7,
+// and 51.5 / 41.4 / 33.7 / 29.7 in 3 / 4 / 6 / 8; F32, 3 x 217 tokens on
+// 897..2,320: 309 unsplit, 168 in parts of at most 20 steps.
+void plan_balanced(const mvr_paged_attention_args* a, const LiveSeqs& live, int64_t n_live, int len_live,
+                   mvr::PagedAttentionPlan& plan) {
+  const int64_t cus = device_cus();
+  const int group = a->num_q_heads / a->num_kv_heads;
+  const int step_keys = prefill_step_keys(a);
+  // fn(tiles, steps per tile) for each sequence of the launch.
+  auto each = [&](auto fn) {
+    if (!live.seq_lens || !live.cu_q_lens) {
+      fn(n_live * a->num_kv_heads * plan.row_tiles, (int64_t)(len_live + step_keys - 1) / step_keys);
+      return;
+    }
+    for (int s = 0; s < a->num_seqs; s++) {
+      const int64_t q = live.cu_q_lens[s + 1] - live.cu_q_lens[s];
+      if (q < live.q_min) continue;
+      fn(a->num_kv_heads * ((group * q + mvr::kPrefillBlockRows - 1) / mvr::kPrefillBlockRows),
+         ((int64_t)live.seq_lens[s] + step_keys - 1) / step_keys);
+    }
+  };
+  int64_t tiles = 0, steps = 0, longest = 0;
+  each([&](int64_t t, int64_t n) {
+    tiles += t;
+    steps += t * n;
+    longest = std::max(longest, n);
+  });
+  if (tiles == 0 || tiles > 4 * cus) return;
+  // Blocks of the call in parts of at most `part` steps, and its longest part.
+  auto blocks_at = [&](int64_t part, int64_t* longest_part = nullptr) {
+    int64_t blocks = 0, most = 0;
+    each([&](int64_t t, int64_t n) {
+      const int64_t parts = std::min<int64_t>((n + part - 1) / part, mvr::kPrefillMaxParts);
+      blocks += t * parts;
+      most = std::max(most, (n + parts - 1) / parts);
+    });
+    if (longest_part) *longest_part = most;
+    return blocks;
+  };
+  const bool f16 = a->dtype == MVR_DTYPE_F16;
+  const size_t slot_bytes = (size_t)mvr::kPrefillBlockRows * (a->head_dim + 2) * sizeof(float);
+  const int64_t slots = (int64_t)(live.prefill_budget / slot_bytes);
+  static const int split_override = env_int("MVR_ATTN_PREFILL_SPLITS", 0);
+  auto cost_us = [&](int64_t blocks, int64_t part) {
+    const double fill = std::min(1.0, (double)blocks / cus);
+    const double step = ((f16 ? 1.5 : 6.9) + (f16 ? 0.5 : 0.9) * fill) * a->head_dim / 128;
+    const double load = blocks <= cus ? (double)part : std::max((double)part, (double)steps / cus + part / 2);
+    return load * step + 8.0 * ((blocks + cus - 1) / cus);
+  };
+  double best = split_override > 1 ? INFINITY : 0.97 * cost_us(tiles, longest);
+  int64_t best_part = 0;
+  for (int64_t quarters : {1, 2, 3, 4, 8, 12, 16}) { // of a block per CU
+    const int64_t most = std::min(split_override > 1 ? tiles * split_override : quarters * cus / 4, slots);
+    if (split_override == 1 || most < tiles) continue;
+    int64_t lo = std::min<int64_t>(2, longest), hi = longest; // blocks_at(hi) = tiles <= most
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) / 2;
+      if (blocks_at(mid) <= most)
+        hi = mid;
+      else
+        lo = mid + 1;
+    }
+    if (lo >= longest) continue;
+    int64_t part = 0;
+    const int64_t blocks = blocks_at(lo, &part);
+    const double cost = cost_us(blocks, part) + 5 + 11.0 * blocks / cus * a->head_dim / 128;
+    if (cost < best) {
+      best = cost;
+      best_part = lo;
+    }
+    if (split_override > 1) break;
+  }
+  // (Part counts are 32-bit on the device, whatever its tables hold.)
+  if (best_part == 0 || (int64_t)a->num_seqs * a->num_kv_heads * plan.row_tiles * mvr::kPrefillMaxParts >= (1LL << 31)) return;
+  plan.part_steps = (int)best_part;
+  plan.balanced_blocks = (int)blocks_at(best_part);
+  plan.balanced_tiles = (int)tiles;
+  // Slots for a block per CU at least: up to there the workspace does not
+  // depend on the lengths.
+  plan.balanced_slots = (int)std::max<int64_t>(plan.balanced_blocks, std::min(cus, slots));
+  const size_t prow = (size_t)plan.balanced_slots * mvr::kPrefillBlockRows;
+  plan.partial_bytes = align_up(prow * a->head_dim * sizeof(float), 256) + align_up(prow * 2 * sizeof(float), 256);
+}
 
 mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_prefill = true,
                                   LiveSeqs live = LiveSeqs{}, bool force_prefill = false) {
@@ -217,18 +324,6 @@ mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_
     plan.prefill = true;
     plan.row_tiles = (int)((rows_max + mvr::kPrefillBlockRows - 1) / mvr::kPrefillBlockRows);
     const int64_t live_blocks = n_live * a->num_kv_heads * plan.row_tiles;
-    const int key_tiles = (len_live + 31) / 32;
-    static const int split_override = env_int("MVR_ATTN_PREFILL_SPLITS", 0);
-    int64_t splits = split_override;
-    if (splits <= 0) {
-      // Split keys only while blocks leave CUs idle: one block per CU ran
-      // faster than two half-length blocks plus the merge pass.
-      splits = (int64_t)device_cus() / live_blocks;
-      if (splits > key_tiles / 8) splits = key_tiles / 8; // keep >= 8 key tiles per split
-    }
-    if (splits > 8) splits = 8; // the merge holds one split per lane; 8 is plenty
-    if (splits < 1) splits = 1;
-    plan.kv_splits = (int)splits;
     // Wavefront groups per block.  Two groups share a block's 128 rows and
     // take alternating key tiles, two wavefronts per SIMD behind one barrier;
     // rows of more than 128 elements take one group (one wavefront per SIMD
@@ -247,12 +342,8 @@ mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_
     else if (groups_override == 1 || groups_override == 2)
       plan.prefill_groups = groups_override;
     else
-      plan.prefill_groups = a->dtype == MVR_DTYPE_F16 && live_blocks * splits >= 4LL * device_cus() ? 1 : 2;
-    if (splits > 1) {
-      const int64_t split_seqs = live.split_count > 0 && live.split_count < a->num_seqs ? live.split_count : a->num_seqs;
-      const size_t prow = (size_t)(split_seqs * a->num_kv_heads * plan.row_tiles) * splits * mvr::kPrefillBlockRows;
-      plan.partial_bytes = align_up(prow * a->head_dim * sizeof(float), 256) + align_up(prow * 2 * sizeof(float), 256);
-    }
+      plan.prefill_groups = a->dtype == MVR_DTYPE_F16 && live_blocks >= 4LL * device_cus() ? 1 : 2;
+    if (plan.prefill_groups == 2 || a->head_dim > 128) plan_balanced(a, live, n_live, len_live, plan);
     return plan;
   }
   plan.row_blocks = rows_max <= 16 || !all_plans ? 1 : 2;
@@ -513,8 +604,7 @@ int launch_planned(const mvr_paged_attention_args* a, const mvr::PagedAttentionP
     f.out_stride_head = a->out_stride_head;
     f.out_stride_token = a->out_stride_token;
     if (plan.partial_bytes) {
-      const size_t prow = (size_t)(cp.seq_count ? cp.seq_count : a->num_seqs) * a->num_kv_heads *
-                          plan.row_tiles * plan.kv_splits * mvr::kPrefillBlockRows;
+      const size_t prow = (size_t)plan.balanced_slots * mvr::kPrefillBlockRows;
       char* w = static_cast<char*>(ws);
       f.partial_o = reinterpret_cast<float*>(w);
       f.partial_ml = reinterpret_cast<float*>(w + align_up(prow * a->head_dim * sizeof(float), 256));
@@ -525,7 +615,9 @@ int launch_planned(const mvr_paged_attention_args* a, const mvr::PagedAttentionP
     f.page_size = a->page_size;
     mvr::page_divider(a->page_size, f.page_magic, f.page_magic_shift);
     f.row_tiles = plan.row_tiles;
-    f.kv_splits = plan.kv_splits;
+    f.balanced_blocks = plan.balanced_blocks;
+    f.part_steps = plan.part_steps;
+    f.balanced_tiles = plan.balanced_tiles;
     f.groups = plan.prefill_groups;
     f.scale_log2 = scale * 1.4426950408889634f;
     f.key_end = cp.key_end;
@@ -611,7 +703,7 @@ int check_workspace(const mvr_paged_attention_args* a, size_t need) {
 //     q_len is at most its planned q_len (qmax);
 //   launch 1, the prefill kernel planned for max_q_len, computing every
 //     sequence that launch 0 does not (outside [lo, hi], or with q_len >
-//     qmax): its main grid (key splits and partial slots included) covers the
+//     qmax): its main grid covers the
 //     range that holds the prefill class, and one catch-up block per
 //     sequence covers the rest of [lo, hi] (each exits at once unless a stale
 //     hint or a wrong guess put a prefill-sized request there, which it then
@@ -623,6 +715,21 @@ int check_workspace(const mvr_paged_attention_args* a, size_t need) {
 // context splits), and a stale hint costs speed, never rows.
 constexpr int kSmallRows = 32;
 
+// The call's host tables for a prefill launch of the sequences with at least
+// q_min new tokens, if both are there and within the call's bounds.
+void prefill_tables(const mvr_paged_attention_args* a, int q_min, LiveSeqs& live) {
+  const int group = a->num_q_heads / a->num_kv_heads;
+  if (!a->cu_q_lens_host || !a->seq_lens_host || (int64_t)group * a->max_q_len <= 64) return;
+  for (int s = 0; s < a->num_seqs; s++) {
+    const int q = a->cu_q_lens_host[s + 1] - a->cu_q_lens_host[s];
+    const int L = a->seq_lens_host[s];
+    if (q < 1 || q > a->max_q_len || L < q || L > a->max_seq_len) return;
+  }
+  live.cu_q_lens = a->cu_q_lens_host;
+  live.seq_lens = a->seq_lens_host;
+  live.q_min = q_min;
+}
+
 struct CallPlan {
   int n = 1;                       // launches (1 or 2)
   mvr_paged_attention_args part[2]; // each launch's view of the call
@@ -632,10 +739,14 @@ struct CallPlan {
   size_t total = 0;
 };
 
-CallPlan make_call_plan(const mvr_paged_attention_args* a) {
+// budget: the largest workspace of the prefill launch's partials.
+CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget) {
   CallPlan c;
   c.part[0] = *a;
-  c.plan[0] = make_plan(a);
+  LiveSeqs all;
+  all.prefill_budget = budget;
+  prefill_tables(a, 1, all);
+  c.plan[0] = make_plan(a, true, all);
   c.total = c.plan[0].partial_bytes;
   const int group = a->num_q_heads / a->num_kv_heads;
   const int small_q = kSmallRows / group; // largest q_len of the small class (0: no such class)
@@ -717,7 +828,8 @@ CallPlan make_call_plan(const mvr_paged_attention_args* a) {
   p1.cu_q_lens_host = nullptr;
   LiveSeqs live1;
   live1.count = count[1];
-  live1.split_count = last[1] - first[1] + 1;
+  live1.prefill_budget = budget;
+  if (hinted) prefill_tables(a, qmax + 1, live1);
   if (hinted) {
     if (sl) live1.max_seq_len = lmax[1];
     p1.sum_seq_lens = sl ? lsum[1] : 0;
@@ -727,18 +839,33 @@ CallPlan make_call_plan(const mvr_paged_attention_args* a) {
   e1.skip_seq_lo = first[0];
   e1.skip_seq_hi = last[0];
   e1.skip_q_max = qmax;
-  if (live1.split_count > 0 && live1.split_count < a->num_seqs) {
+  const int span1 = last[1] - first[1] + 1;
+  if (span1 < a->num_seqs && c.plan[1].balanced_blocks == 0) {
     // Main grid over the prefill range; the rest of the decode range gets a
     // catch-up block per sequence (it exits unless a stale hint put a
-    // prefill-sized request there).
+    // prefill-sized request there).  (A balanced grid finds every sequence
+    // that launch 0 leaves by itself.)
     e1.seq_lo = first[1];
-    e1.seq_count = (int32_t)live1.split_count;
+    e1.seq_count = span1;
     e1.catch_lo = first[0];
     e1.catch_count = last[0] - first[0] + 1;
   }
   c.offset[0] = 0;
   c.offset[1] = align_up(c.plan[0].partial_bytes, 256);
   c.total = c.offset[1] + c.plan[1].partial_bytes;
+  return c;
+}
+
+// The call's plan in `limit` bytes of workspace, `used` of them taken: where
+// the balanced prefill grid's partials do not fit, it gets fewer blocks, down
+// to none (the unsplit grid, which needs no workspace).
+CallPlan make_call_plan(const mvr_paged_attention_args* a, size_t limit = SIZE_MAX, size_t used = 0) {
+  CallPlan c = plan_call_within(a, LiveSeqs{}.prefill_budget);
+  const mvr::PagedAttentionPlan& last = c.plan[c.n - 1];
+  if (last.prefill && used + c.total > limit) {
+    const size_t other = used + c.total - last.partial_bytes + 512; // alignment of the two partial arrays
+    c = plan_call_within(a, limit > other ? limit - other : 0);
+  }
   return c;
 }
 
@@ -787,7 +914,7 @@ bool needs_repack(const mvr_paged_attention_args* a) {
   return false;
 }
 
-RepackPlan make_repack_plan(const mvr_paged_attention_args* a, char* ws) {
+RepackPlan make_repack_plan(const mvr_paged_attention_args* a, char* ws, size_t limit = SIZE_MAX) {
   RepackPlan r;
   r.pages16 = (a->max_seq_len + mvr::kChunkTokens - 1) / mvr::kChunkTokens;
   const int es = a->dtype == MVR_DTYPE_F16 ? 2 : 4;
@@ -802,7 +929,7 @@ RepackPlan make_repack_plan(const mvr_paged_attention_args* a, char* ws) {
   r.a16.key_pool = ws;
   r.a16.value_pool = ws ? ws + off_v : nullptr;
   r.a16.block_tables = ws ? reinterpret_cast<const int32_t*>(ws + off_bt) : nullptr;
-  r.call = make_call_plan(&r.a16);
+  r.call = make_call_plan(&r.a16, limit, r.off_part);
   r.total = r.off_part + r.call.total;
   return r;
 }
@@ -1123,9 +1250,10 @@ static void* noalloc_scratch() {
 // The launches of one mvr_paged_attention call on the workspace the
 // arguments carry (scalar checks already done).
 static int paged_attention_launches(const mvr_paged_attention_args* a) {
+  const size_t limit = a->workspace ? a->workspace_bytes : 0;
   int rc;
   if (needs_repack(a)) {
-    const RepackPlan r = make_repack_plan(a, static_cast<char*>(a->workspace));
+    const RepackPlan r = make_repack_plan(a, static_cast<char*>(a->workspace), limit);
     rc = check_workspace(a, r.total);
     if (rc != MVR_OK) return rc;
     const int es = a->dtype == MVR_DTYPE_F16 ? 2 : 4;
@@ -1137,7 +1265,7 @@ static int paged_attention_launches(const mvr_paged_attention_args* a) {
     if (err != hipSuccess) return fail(MVR_E_HIP, "kernel launch failed: %s", hipGetErrorString(err));
     return launch_call(r.call, static_cast<char*>(a->workspace) + r.off_part);
   }
-  const CallPlan c = make_call_plan(a);
+  const CallPlan c = make_call_plan(a, limit);
   rc = check_workspace(a, c.total);
   if (rc != MVR_OK) return rc;
   return launch_call(c, static_cast<char*>(a->workspace));
@@ -1157,13 +1285,13 @@ int mvr_paged_attention_noalloc(const mvr_paged_attention_args* a) {
   g_last_error[0] = 0;
   int rc = check_scalars(a);
   if (rc != MVR_OK) return rc;
-  const size_t need =
-      needs_repack(a) ? make_repack_plan(a, nullptr).total : make_call_plan(a).total;
-  if (need > (size_t)MVR_NOALLOC_SCRATCH_BYTES)
+  constexpr size_t limit = MVR_NOALLOC_SCRATCH_BYTES;
+  const size_t need = needs_repack(a) ? make_repack_plan(a, nullptr, limit).total : make_call_plan(a, limit).total;
+  if (need > limit)
     return fail(MVR_E_WORKSPACE,
                 "this call needs %zu bytes of scratch, more than the %zu bytes of the library's static scratch; "
                 "call mvr_paged_attention with a workspace instead",
-                need, (size_t)MVR_NOALLOC_SCRATCH_BYTES);
+                need, limit);
   mvr_paged_attention_args b = *a;
   b.workspace = nullptr;
   b.workspace_bytes = 0;

@@ -29,8 +29,9 @@
 //     from the S^T registers;  O^T += V^T P^T in D/16 MFMAs.
 // Blocks of one (sequence, KV head) are mapped onto one XCD (workgroups are
 // dispatched round-robin over the 8 XCDs), so their shared K/V stays in that
-// XCD's L2.  The key range can be split (kv_splits) to fill the device; split
-// results go to an fp32 partial workspace that prefill_merge_kernel combines.
+// XCD's L2.  Grids of few or unequal tiles run balanced instead: each tile's
+// keys in parts of about one length, a block per part, combined by
+// prefill_merge_kernel from an fp32 partial workspace.
 #include "paged_prefill.hpp"
 
 #include <math.h>
@@ -44,6 +45,7 @@ typedef _Float16 half_t;
 typedef half_t half8 __attribute__((ext_vector_type(8)));
 typedef half_t half4 __attribute__((ext_vector_type(4)));
 typedef short short4v __attribute__((ext_vector_type(4)));
+typedef float float2v __attribute__((ext_vector_type(2)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -62,6 +64,7 @@ constexpr int kBlockRows = kRowsPerWave * kRowWaves;
 // SIMD).
 constexpr int kMergeWaves = 4; // wavefronts per block of prefill_merge_kernel
 constexpr int kXcds = 8;
+constexpr int kMaxParts = kPrefillMaxParts;
 #ifndef MVR_PREFILL_STAGES
 #define MVR_PREFILL_STAGES 2
 #endif
@@ -109,27 +112,38 @@ __device__ __forceinline__ void tile_barrier() {
   asm volatile("" ::: "memory");
 }
 
-__device__ __forceinline__ SeqRows load_rows(const PrefillParams& p, int b) {
+__device__ __forceinline__ SeqRows make_rows(const PrefillParams& p, int b, int seq_len, int q_start, int q_end, int key_end) {
   SeqRows s;
   // single_seq_len is the call's max_seq_len (its pages fit a block-table row,
   // checked on the host): a larger device seq_len is clamped to it.
-  s.seq_len = p.seq_lens ? min(p.seq_lens[b], p.single_seq_len) : p.single_seq_len;
-  if (p.cu_q_lens) {
-    s.q_start = p.cu_q_lens[b];
-    s.q_len = p.cu_q_lens[b + 1] - s.q_start;
-  } else {
-    s.q_start = 0;
-    s.q_len = p.single_q_len;
-  }
+  s.seq_len = p.seq_lens ? min(seq_len, p.single_seq_len) : p.single_seq_len;
+  s.q_start = p.cu_q_lens ? q_start : 0;
+  s.q_len = p.cu_q_lens ? q_end - q_start : p.single_q_len;
   // Another launch's sequence: no rows here (its blocks exit at once).
   if (s.q_len <= p.skip_q_max && b >= p.skip_seq_lo && b <= p.skip_seq_hi) s.q_len = 0;
   if (p.key_end) { // cascade prefix pass: every row sees every key before key_end
-    s.key_end = p.key_end[b];
-    s.seq_len = s.key_end + s.q_len;
+    s.key_end = key_end;
+    s.seq_len = key_end + s.q_len;
   } else {
     s.key_end = s.seq_len;
   }
   return s;
+}
+
+__device__ __forceinline__ SeqRows load_rows(const PrefillParams& p, int b) {
+  return make_rows(p, b, p.seq_lens ? p.seq_lens[b] : 0, p.cu_q_lens ? p.cu_q_lens[b] : 0,
+                   p.cu_q_lens ? p.cu_q_lens[b + 1] : 0, p.key_end ? p.key_end[b] : 0);
+}
+
+// One sequence per lane: the tables' loads, an absent table's from one that is
+// there, go out together (one after the other, each waits for a round trip).
+__device__ __forceinline__ SeqRows load_lane_rows(const PrefillParams& p, int b) {
+  const int32_t* any = p.block_tables;
+  const int seq_len = *(p.seq_lens ? p.seq_lens + b : any);
+  const int q_start = *(p.cu_q_lens ? p.cu_q_lens + b : any);
+  const int q_end = *(p.cu_q_lens ? p.cu_q_lens + b + 1 : any);
+  const int key_end = *(p.key_end ? p.key_end + b : any);
+  return make_rows(p, b, seq_len, q_start, q_end, key_end);
 }
 
 // Causal limit of query i within this call's keys (common.rs:948-965).
@@ -179,11 +193,13 @@ struct Tile {
   __device__ static __forceinline__ int kswz(int t) { return t & (kSwzGroup - 1); }
 };
 
-// One (sequence, kv head, 128-row tile, key split): each step stages one
-// key tile per group, then QK^T, softmax and PV in turn.
+// Steps [step0, step1) of one (sequence, kv head, 128-row tile); a step is one
+// key tile per group: it stages them, then QK^T, softmax and PV in turn.  Steps
+// past the tile's last visible key are left out.  A part (not all of the
+// tile's steps) writes its unnormalised rows to partial slot `slot`.
 template <int D, typename T, int TT, int G, bool TP>
 __device__ __forceinline__ void prefill_tile_serial(const PrefillParams& p, const SeqRows& s, int b, int h, int rt,
-                                                    int split, int kv_splits) {
+                                                    int step0, int step1, int slot) {
   static_assert(G == 1 || G == 2, "one or two wavefront groups");
   typedef Tile<D, T, TT, G> TL;
   constexpr bool kF32 = TL::kF32;
@@ -215,12 +231,10 @@ __device__ __forceinline__ void prefill_tile_serial(const PrefillParams& p, cons
 
   const int rows = p.group_size * s.q_len;
   const int n_tiles = block_key_tiles<TT>(s, p.group_size, rt);
-  if (n_tiles == 0) return; // whole block: uniform return before any barrier
-  const int tiles_per_split = (n_tiles + kv_splits - 1) / kv_splits;
-  const int j0 = split * tiles_per_split;
-  const int j1 = min(j0 + tiles_per_split, n_tiles);
-  const int64_t slot =
-      (int64_t)(((b - p.seq_lo) * p.num_kv_heads + h) * p.row_tiles + rt) * p.kv_splits + split; // kv_splits > 1
+  const int j0 = G * step0;
+  if (j0 >= n_tiles) return; // whole block: uniform return before any barrier
+  const int j1 = min(G * step1, n_tiles);
+  const bool partial = step0 > 0 || j1 < n_tiles;
 
   // This lane's query row.
   const int rho = rt * kBlockRows + rw * kRowsPerWave + (l & 31);
@@ -699,6 +713,23 @@ __device__ __forceinline__ void prefill_tile_serial(const PrefillParams& p, cons
   }
 
   const float ltot = lsum + __shfl_xor(lsum, 32);
+  if (partial) {
+    // As the registers lie, [row wavefront][n][e / 4][lane] float4: 1 KiB per
+    // store.  (Written as rows, a store touches 32 rows 32 bytes at a time.)
+    float4v* dst = reinterpret_cast<float4v*>(p.partial_o) + ((int64_t)slot * kRowWaves + rw) * (D / 8 * 64) + l;
+#pragma unroll
+    for (int n = 0; n < D / 32; n++)
+#pragma unroll
+      for (int a = 0; a < 4; a++)
+        dst[(n * 4 + a) * 64] = float4v{o[n][4 * a], o[n][4 * a + 1], o[n][4 * a + 2], o[n][4 * a + 3]};
+    if (hh == 0) {
+      // m is kept in log2 units of the scaled score, as the decode partials.
+      float* ml = p.partial_ml + ((int64_t)slot * kBlockRows + rw * kRowsPerWave + l) * 2;
+      ml[0] = m;
+      ml[1] = ltot;
+    }
+    return;
+  }
   if constexpr (kF32) {
     // Lane holds O^T[d][rho] for d = (D/32)*(8*(e/4) + 4*hh + e%4) + n.
     auto put = [&](float* dst, float scale) {
@@ -717,14 +748,7 @@ __device__ __forceinline__ void prefill_tile_serial(const PrefillParams& p, cons
       }
     };
     if (!valid) return;
-    if (kv_splits > 1) {
-      const int64_t prow = slot * kBlockRows + rw * kRowsPerWave + (l & 31);
-      put(p.partial_o + prow * D, 1.f);
-      if (hh == 0) {
-        p.partial_ml[prow * 2 + 0] = m;
-        p.partial_ml[prow * 2 + 1] = ltot;
-      }
-    } else if (p.state_o) {
+    if (p.state_o) {
       const int64_t srow = (int64_t)(h * p.group_size + r) * p.state_tokens + s.q_start + i;
       put(p.state_o + srow * D, 1.f / ltot);
       if (hh == 0) p.state_lse[srow] = m + __log2f(ltot);
@@ -736,95 +760,79 @@ __device__ __forceinline__ void prefill_tile_serial(const PrefillParams& p, cons
     return;
   }
   // Lane holds O^T[d][rho] for d = 32n + 8*(e/4) + 4*hh + e%4.
-  if (kv_splits == 1) {
-    if (valid && p.state_o) {
-      const float inv = 1.f / ltot;
-      const int64_t srow = (int64_t)(h * p.group_size + r) * p.state_tokens + s.q_start + i;
-      float* dst = p.state_o + srow * D;
-#pragma unroll
-      for (int n = 0; n < D / 32; n++)
-#pragma unroll
-        for (int a = 0; a < 4; a++)
-          *reinterpret_cast<float4v*>(dst + 32 * n + 8 * a + 4 * hh) =
-              float4v{o[n][4 * a], o[n][4 * a + 1], o[n][4 * a + 2], o[n][4 * a + 3]} * inv;
-      if (hh == 0) p.state_lse[srow] = m + __log2f(ltot);
-    } else if (!p.state_o) {
-      // The wavefront's 32 rows go through LDS (its own 32 x D slice of the
-      // idle V stage 0: the hand-off used K stages 0 and 1 only), so that the
-      // output is written 16 bytes per lane along whole rows.  Written
-      // straight from the MFMA layout, each store instruction would touch 32
-      // rows 8 bytes at a time: 3.6 of the 47 us of the Qwen2-7B prefill
-      // chunk.  The slice swizzles 16-byte chunks with the row (chunk ^ row %
-      // chunks), so neither the 8-byte writes nor the 16-byte reads collide
-      // in LDS banks.  A wavefront's LDS accesses complete in order, so its
-      // reads see its writes.  (Head dimensions whose rows do not tile a
-      // wavefront's 64 lanes in whole 16-byte chunks, or whose V stage is
-      // too small or carries part of the hand-off, store straight from the
-      // MFMA layout.)
-      constexpr int kChunksPerRow = D / 8;
-      constexpr bool kStaged = 64 % kChunksPerRow == 0 && kRowWaves * kRowsPerWave * D <= TL::kElems &&
-                               (D / 32) * kRowWaves * 1024 <= 2 * kStageFloats;
-      if constexpr (!kStaged) {
-        if (valid) {
-          const float inv = 1.f / ltot;
-          half_t* dst = static_cast<half_t*>(p.out) + (int64_t)(h * p.group_size + r) * p.out_stride_head +
-                        (int64_t)(s.q_start + i) * p.out_stride_token;
-#pragma unroll
-          for (int n = 0; n < D / 32; n++)
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-              *reinterpret_cast<half4*>(dst + 32 * n + 8 * a + 4 * hh) =
-                  half4{(half_t)(o[n][4 * a] * inv), (half_t)(o[n][4 * a + 1] * inv), (half_t)(o[n][4 * a + 2] * inv),
-                        (half_t)(o[n][4 * a + 3] * inv)};
-        }
-      } else {
-        half_t* slice = reinterpret_cast<half_t*>(v_lds0) + rw * kRowsPerWave * D;
-        const float inv = valid ? 1.f / ltot : 0.f;
-        const int row = l & 31;
-#pragma unroll
-        for (int n = 0; n < D / 32; n++)
-#pragma unroll
-          for (int a = 0; a < 4; a++) {
-            const half4 v4 = {(half_t)(o[n][4 * a] * inv), (half_t)(o[n][4 * a + 1] * inv),
-                              (half_t)(o[n][4 * a + 2] * inv), (half_t)(o[n][4 * a + 3] * inv)};
-            const int chunk = (4 * n + a) ^ (row & (kChunksPerRow - 1));
-            *reinterpret_cast<half4*>(slice + row * D + chunk * 8 + 4 * hh) = v4;
-          }
-        constexpr int kRowsPerRead = 64 / kChunksPerRow;
-        // The lane index is opaque to the optimiser here, so the read offsets
-        // below are computed where they are used, not hoisted to the kernel's
-        // entry, where (in the catch-up loop) they were spilled to a private
-        // segment.
-        int le = l;
-        asm volatile("" : "+v"(le));
-        const int cc = le % kChunksPerRow;
-#pragma unroll
-        for (int k = 0; k < kRowsPerWave / kRowsPerRead; k++) {
-          const int rr = k * kRowsPerRead + le / kChunksPerRow; // row of the wavefront's 32
-          const half8 v8 = *reinterpret_cast<const half8*>(slice + rr * D + (cc ^ (rr & (kChunksPerRow - 1))) * 8);
-          const int rho_w = rt * kBlockRows + rw * kRowsPerWave + rr;
-          if (rho_w < rows) {
-            const int rr_r = rho_w / s.q_len, rr_i = rho_w % s.q_len;
-            half_t* dst = static_cast<half_t*>(p.out) + (int64_t)(h * p.group_size + rr_r) * p.out_stride_head +
-                          (int64_t)(s.q_start + rr_i) * p.out_stride_token;
-            *reinterpret_cast<half8*>(dst + cc * 8) = v8;
-          }
-        }
-      }
-    }
-  } else if (valid) {
-    const int64_t prow = slot * kBlockRows + rw * kRowsPerWave + (l & 31);
-    float* dst = p.partial_o + prow * D;
+  if (valid && p.state_o) {
+    const float inv = 1.f / ltot;
+    const int64_t srow = (int64_t)(h * p.group_size + r) * p.state_tokens + s.q_start + i;
+    float* dst = p.state_o + srow * D;
 #pragma unroll
     for (int n = 0; n < D / 32; n++)
 #pragma unroll
       for (int a = 0; a < 4; a++)
         *reinterpret_cast<float4v*>(dst + 32 * n + 8 * a + 4 * hh) =
-            float4v{o[n][4 * a], o[n][4 * a + 1], o[n][4 * a + 2], o[n][4 * a + 3]};
-    if (hh == 0) {
-      // m is kept in log2 units of the scaled score, as the decode partials.
-      p.partial_ml[prow * 2 + 0] = m;
-      p.partial_ml[prow * 2 + 1] = ltot;
+            float4v{o[n][4 * a], o[n][4 * a + 1], o[n][4 * a + 2], o[n][4 * a + 3]} * inv;
+    if (hh == 0) p.state_lse[srow] = m + __log2f(ltot);
+  } else if (!p.state_o) {
+    // The wavefront's 32 rows go through LDS (its own 32 x D slice of the
+    // idle V stage 0: the hand-off used K stages 0 and 1 only), so that the
+    // output is written 16 bytes per lane along whole rows.  Written
+    // straight from the MFMA layout, each store instruction would touch 32
+    // rows 8 bytes at a time: 3.6 of the 47 us of the Qwen2-7B prefill
+    // chunk.  The slice swizzles 16-byte chunks with the row (chunk ^ row %
+    // chunks), so neither the 8-byte writes nor the 16-byte reads collide
+    // in LDS banks.  A wavefront's LDS accesses complete in order, so its
+    // reads see its writes.  (Head dimensions whose rows do not tile a
+    // wavefront's 64 lanes in whole 16-byte chunks, or whose V stage is
+    // too small or carries part of the hand-off, store straight from the
+    // MFMA layout.)
+    constexpr int kChunksPerRow = D / 8;
+    constexpr bool kStaged = 64 % kChunksPerRow == 0 && kRowWaves * kRowsPerWave * D <= TL::kElems &&
+                             (D / 32) * kRowWaves * 1024 <= 2 * kStageFloats;
+    if constexpr (!kStaged) {
+      if (valid) {
+        const float inv = 1.f / ltot;
+        half_t* dst = static_cast<half_t*>(p.out) + (int64_t)(h * p.group_size + r) * p.out_stride_head +
+                      (int64_t)(s.q_start + i) * p.out_stride_token;
+#pragma unroll
+        for (int n = 0; n < D / 32; n++)
+#pragma unroll
+          for (int a = 0; a < 4; a++)
+            *reinterpret_cast<half4*>(dst + 32 * n + 8 * a + 4 * hh) =
+                half4{(half_t)(o[n][4 * a] * inv), (half_t)(o[n][4 * a + 1] * inv), (half_t)(o[n][4 * a + 2] * inv),
+                      (half_t)(o[n][4 * a + 3] * inv)};
+      }
+    } else {
+      half_t* slice = reinterpret_cast<half_t*>(v_lds0) + rw * kRowsPerWave * D;
+      const float inv = valid ? 1.f / ltot : 0.f;
+      const int row = l & 31;
+#pragma unroll
+      for (int n = 0; n < D / 32; n++)
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+          const half4 v4 = {(half_t)(o[n][4 * a] * inv), (half_t)(o[n][4 * a + 1] * inv),
+                            (half_t)(o[n][4 * a + 2] * inv), (half_t)(o[n][4 * a + 3] * inv)};
+          const int chunk = (4 * n + a) ^ (row & (kChunksPerRow - 1));
+          *reinterpret_cast<half4*>(slice + row * D + chunk * 8 + 4 * hh) = v4;
+        }
+      constexpr int kRowsPerRead = 64 / kChunksPerRow;
+      // The lane index is opaque to the optimiser here, so the read offsets
+      // below are computed where they are used, not hoisted to the kernel's
+      // entry, where (in the catch-up loop) they were spilled to a private
+      // segment.
+      int le = l;
+      asm volatile("" : "+v"(le));
+      const int cc = le % kChunksPerRow;
+#pragma unroll
+      for (int k = 0; k < kRowsPerWave / kRowsPerRead; k++) {
+        const int rr = k * kRowsPerRead + le / kChunksPerRow; // row of the wavefront's 32
+        const half8 v8 = *reinterpret_cast<const half8*>(slice + rr * D + (cc ^ (rr & (kChunksPerRow - 1))) * 8);
+        const int rho_w = rt * kBlockRows + rw * kRowsPerWave + rr;
+        if (rho_w < rows) {
+          const int rr_r = rho_w / s.q_len, rr_i = rho_w % s.q_len;
+          half_t* dst = static_cast<half_t*>(p.out) + (int64_t)(h * p.group_size + rr_r) * p.out_stride_head +
+                        (int64_t)(s.q_start + rr_i) * p.out_stride_token;
+          *reinterpret_cast<half8*>(dst + cc * 8) = v8;
+        }
+      }
     }
   }
 }
@@ -838,27 +846,147 @@ constexpr int prefill_tile_tokens() {
   return sizeof(T) == 4 ? 32 : 64;
 }
 
-// Main grid: block x covers (sequence, kv head, row tile, key split) of the
-// main range.  XCD-aware decode: block x runs on XCD x % 8 and all blocks of
-// one (sequence, kv head) pair sit on the same XCD, so their shared K/V stays
-// in that XCD's L2 (with fewer pairs than XCDs, plain linear order keeps
-// every XCD busy).  Catch-up blocks follow the main grid.
-template <int D, typename T, int G, bool TP>
-__device__ __forceinline__ void prefill_tile(const PrefillParams& p, const SeqRows& s, int b, int h, int rt, int split,
-                                             int kv_splits) {
-  prefill_tile_serial<D, T, prefill_tile_tokens<D, T>(), G, TP>(p, s, b, h, rt, split, kv_splits);
+// ---------------------------------------------------------------------------
+// Balanced grid: one block per part, a part being an even share, of at most
+// part_steps steps, of one row tile's keys (a step is G TT keys).
+// ---------------------------------------------------------------------------
+// Sequence b holds num_kv_heads x (its row tiles) tiles of the same number of
+// parts (from its longest row; rows with an earlier causal limit split their
+// own steps as many ways), in (sequence, kv head, part, row tile) order.
+// Everything comes from the device length tables: a block finds its part with
+// one wave-wide scan per 64 sequences, whatever the host planned from.  Tables
+// that give more parts or tiles than the host planned for (a stale hint) are
+// not split at all: the blocks then stride over whole tiles.
+// (Equal runs of steps, cutting tiles wherever a run ends, balance better but
+// give most blocks two tiles, and a tile costs about 9 us beside its steps:
+// 34 against 24 us on a 256-token chunk behind 2,048 tokens, F16, and 173
+// against 167 us on three ragged F32 chunks.)
+
+// Inclusive sum over the wavefront's lanes: rows of 16 by shifts, then each
+// row's last lane into the rows after it (DPP, no LDS round trips).
+__device__ __forceinline__ int wave_inclusive_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false); // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false); // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false); // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false); // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false); // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false); // row_bcast:31 into rows 2 and 3
+  return v;
 }
 
+__device__ __forceinline__ int seq_row_tiles(const PrefillParams& p, const SeqRows& s) {
+  return min((p.group_size * s.q_len + kBlockRows - 1) / kBlockRows, p.row_tiles);
+}
+
+// Whether a wavefront looks for parts (the main launch) or for tiles (the merge).
+enum class Find { kPart, kTile };
+
+struct PartPos {
+  SeqRows s;
+  int b, h, rt, part, parts, slot0; // slot0: the slot of the tile's part 0; part j's is slot0 + j * row tiles
+};
+
+// 64 sequences from b0 on, one per lane: the parts of each, their inclusive
+// sum and total (nothing past the last sequence or for another launch's).
+template <int TT, int G>
+struct SeqParts {
+  SeqRows s;
+  int per_tile, tiles, incl, total, tiles_incl;
+  __device__ __forceinline__ SeqParts(const PrefillParams& p, int b0, bool split) : per_tile(0), tiles(0) {
+    const int b = b0 + (int)(threadIdx.x & 63);
+    s = load_lane_rows(p, min(b, p.num_seqs - 1));
+    if (b < p.num_seqs && s.q_len > 0 && s.key_end > 0) {
+      tiles = p.num_kv_heads * seq_row_tiles(p, s);
+      const int steps = (s.key_end + G * TT - 1) / (G * TT);
+      per_tile = split ? min((int)((unsigned)(steps + p.part_steps - 1) / (unsigned)p.part_steps), kMaxParts) : 1;
+    }
+    incl = wave_inclusive_sum(per_tile * tiles);
+    total = __builtin_amdgcn_readlane(incl, 63);
+    tiles_incl = wave_inclusive_sum(tiles);
+  }
+};
+
+// The call's parts; the first 64 sequences' stay in registers.
+template <int TT, int G>
+class CallParts {
+  bool split_;
+  SeqParts<TT, G> head_;
+  int total_, tiles_;
+  __device__ __forceinline__ void sum(const PrefillParams& p) {
+    total_ = head_.total;
+    tiles_ = lane(head_.tiles_incl, 63);
+    for (int b0 = 64; b0 < p.num_seqs; b0 += 64) {
+      const SeqParts<TT, G> c(p, b0, split_);
+      total_ += c.total;
+      tiles_ += lane(c.tiles_incl, 63);
+    }
+  }
+  __device__ __forceinline__ static int lane(int v, int src) { return __builtin_amdgcn_readlane(v, src); }
+
+ public:
+  __device__ __forceinline__ explicit CallParts(const PrefillParams& p) : split_(true), head_(p, 0, true) {
+    sum(p);
+    if (total_ > p.balanced_blocks || tiles_ > p.balanced_tiles) {
+      split_ = false;
+      head_ = SeqParts<TT, G>(p, 0, false);
+      sum(p);
+    }
+  }
+  __device__ __forceinline__ bool split() const { return split_; }
+  // Part i, or (kTile) part 0 of tile i; false past the last one.
+  template <Find kFind>
+  __device__ __forceinline__ bool find(const PrefillParams& p, int i, PartPos& w) const {
+    int slot = 0;
+    for (int b0 = 0; b0 < p.num_seqs; b0 += 64) {
+      const SeqParts<TT, G> c = b0 == 0 ? head_ : SeqParts<TT, G>(p, b0, split_);
+      const int incl = kFind == Find::kPart ? c.incl : c.tiles_incl;
+      const int n = kFind == Find::kPart ? c.per_tile * c.tiles : c.tiles;
+      const int total = lane(incl, 63);
+      if (i < total) {
+        const int src = __builtin_ctzll(__ballot(i < incl));
+        const int rel = i - lane(incl - n, src);
+        w.s = SeqRows{lane(c.s.seq_len, src), lane(c.s.q_start, src), lane(c.s.q_len, src), lane(c.s.key_end, src)};
+        w.b = b0 + src;
+        w.parts = lane(c.per_tile, src);
+        const int rts = seq_row_tiles(p, w.s);
+        if (kFind == Find::kPart) {
+          w.h = (unsigned)rel / (unsigned)(w.parts * rts);
+          const int in_head = rel - w.h * w.parts * rts;
+          w.part = (unsigned)in_head / (unsigned)rts;
+          w.rt = in_head - w.part * rts;
+        } else {
+          w.h = (unsigned)rel / (unsigned)rts;
+          w.part = 0;
+          w.rt = rel - w.h * rts;
+        }
+        w.slot0 = slot + lane(c.incl - c.per_tile * c.tiles, src) + w.h * w.parts * rts + w.rt;
+        return true;
+      }
+      i -= total;
+      slot += c.total;
+    }
+    return false;
+  }
+};
+
+// Main grid: block x covers (sequence, kv head, row tile) of the main range,
+// unsplit.  XCD-aware decode: block x runs on XCD x % 8 and all blocks of one
+// (sequence, kv head) pair sit on the same XCD, so their shared K/V stays in
+// that XCD's L2 (with fewer pairs than XCDs, plain linear order keeps every
+// XCD busy).  Catch-up blocks follow the main grid.
 __host__ __device__ __forceinline__ int64_t prefill_main_blocks(const PrefillParams& p) {
   const int64_t pairs = (int64_t)(p.seq_count ? p.seq_count : p.num_seqs) * p.num_kv_heads;
-  const int64_t per_pair = (int64_t)p.row_tiles * p.kv_splits;
+  const int64_t per_pair = p.row_tiles;
   return pairs >= kXcds ? kXcds * ((pairs + kXcds - 1) / kXcds) * per_pair : pairs * per_pair;
 }
+
+constexpr int kAllSteps = 1 << 24; // past every tile's last step
 
 // TP: pages that are not a multiple of 16 tokens, read in place (head_dim 64
 // and 128; the page size a multiple of the tokens one load covers).
 template <int D, typename T, int G, bool TP>
 __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) void paged_prefill_kernel(PrefillParams p) {
+  constexpr int TT = prefill_tile_tokens<D, T>();
   const int x = blockIdx.x;
   const int main_seqs = p.seq_count ? p.seq_count : p.num_seqs;
   const int main_blocks = (int)prefill_main_blocks(p);
@@ -870,12 +998,12 @@ __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) vo
     if (s.q_len <= 0) return;
     for (int h = 0; h < p.num_kv_heads; h++)
       for (int rt = 0; rt < p.row_tiles; rt++) {
-        prefill_tile<D, T, G, TP>(p, s, b, h, rt, 0, 1);
+        prefill_tile_serial<D, T, TT, G, TP>(p, s, b, h, rt, 0, kAllSteps, 0);
         __syncthreads(); // group 0's hand-off reads end before the next tile refills the stages
       }
     return;
   }
-  const int per_pair = p.row_tiles * p.kv_splits;
+  const int per_pair = p.row_tiles;
   const int pairs = main_seqs * p.num_kv_heads;
   int pair, local;
   if (pairs >= kXcds) {
@@ -889,7 +1017,6 @@ __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) vo
   if (pair >= pairs) return;
   const int h = pair % p.num_kv_heads;
   const int b = p.seq_lo + pair / p.num_kv_heads;
-  const int split = local % p.kv_splits;
   const SeqRows s = load_rows(p, b);
   // Longest first: a tile's causal key range grows with the query positions
   // of its rows, so the pair's tiles are dispatched in decreasing order of
@@ -904,151 +1031,173 @@ __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) vo
   // 667.7 -> 632.6 -> 517.4; chunks on a long prefix level.
   int rt;
   {
-    const int idx = local / p.kv_splits;
     const int tq = s.q_len / kBlockRows; // tiles per query head
     if (s.q_len > 0 && s.q_len % kBlockRows == 0) {
-      rt = idx < p.group_size * tq ? (idx % p.group_size) * tq + (tq - 1 - idx / p.group_size) : idx;
+      rt = local < p.group_size * tq ? (local % p.group_size) * tq + (tq - 1 - local / p.group_size) : local;
     } else {
-      rt = p.row_tiles - 1 - idx;
+      rt = p.row_tiles - 1 - local;
     }
   }
-  prefill_tile<D, T, G, TP>(p, s, b, h, rt, split, p.kv_splits);
+  prefill_tile_serial<D, T, TT, G, TP>(p, s, b, h, rt, 0, kAllSteps, 0);
 }
 
-// Merges the kv_splits partial results of every block tile:
-//   out = sum_j 2^(m_j - M) o_j / sum_j 2^(m_j - M) l_j.
-// One wavefront per merge_rows<D>() output rows of a tile (a 256-thread
-// block covers 4 x that many rows): lane j holds split j's weight, broadcast
-// by readlane.  Every split slot's (m, l) and partial row for all of the
-// wavefront's rows are loaded at once, before the rows' bounds are known
-// (the slots exist for all kv_splits <= kMaxSplits; those of splits that did
-// not run are loaded and never used), so the wavefront costs one round trip.
-// Empty splits (no visible key) hold m = -inf, l = 0 and weigh nothing.
-constexpr int kMaxSplits = 8; // the planner's cap on kv_splits
-// Output rows per wavefront.  Measured on key-split prefill calls: at D=64 (one
-// element per lane) two rows per wavefront took a Qwen2-0.5B-shape chunk from
-// 34.5 to 32.5 us; at D=128 two or four rows slowed the shared-prompt
-// cascade's prefix pass by 1-4 us, so it keeps one.
-template <int D>
-constexpr int merge_rows() {
-  return D == 64 ? 2 : 1;
+// One part of the balanced grid per block (blocks past the last exit; an
+// unsplit call's blocks stride over its tiles).  The parts of one kv head
+// share K/V, so each XCD (block x runs on XCD x % 8) takes consecutive ones
+// where the grid is a multiple of 8.
+template <int D, typename T, int G, bool TP>
+__global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) void paged_prefill_balanced_kernel(
+    PrefillParams p) {
+  constexpr int TT = prefill_tile_tokens<D, T>();
+  const int n = p.balanced_blocks;
+  const int x = n % kXcds == 0 ? (int)(blockIdx.x % kXcds) * (n / kXcds) + (int)(blockIdx.x / kXcds) : (int)blockIdx.x;
+  for (int i = x;; i += n) {
+    // (Scanned again for each of an unsplit call's tiles: kept over the tile,
+    // its lanes' values would spill.)
+    const CallParts<TT, G> parts(p);
+    const bool more = !parts.split();
+    PartPos w;
+    if (!parts.template find<Find::kPart>(p, i, w)) return;
+    const int own = (block_key_tiles<TT>(w.s, p.group_size, w.rt) + G - 1) / G; // steps the tile's rows see
+    const int k = min(w.parts, own);
+    if (w.part < k)
+      prefill_tile_serial<D, T, TT, G, TP>(p, w.s, w.b, w.h, w.rt, (unsigned)(w.part * own) / (unsigned)k,
+                                           (unsigned)((w.part + 1) * own) / (unsigned)k,
+                                           w.slot0 + w.part * seq_row_tiles(p, w.s));
+    if (!more) return;
+    __syncthreads(); // group 0's hand-off reads end before the next tile refills the stages
+  }
 }
-template <int D, typename T, int TT>
-__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
-  // Output elements per lane: D/64 over the wavefront, or, where D is not a
-  // multiple of 64, D/32 over lanes 0..31 (the others hold split weights
-  // only: they re-read lane 31's elements and store nothing).
-  constexpr int kPer = D % 64 == 0 ? D / 64 : D / 32;
-  constexpr int kDimLanes = D / kPer;
-  constexpr int kMergeRows = merge_rows<D>();
-  constexpr int kBlocksPerTile = kBlockRows / (kMergeWaves * kMergeRows);
-  const int tile = blockIdx.x / kBlocksPerTile; // (b - seq_lo, h, rt)
-  const int lr0 = ((blockIdx.x % kBlocksPerTile) * kMergeWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) *
-                  kMergeRows;
+
+// Merges the parts of the balanced grid's tiles:
+//   out = sum_j 2^(m_j - M) o_j / sum_j 2^(m_j - M) l_j,  M = max_j m_j.
+// A wavefront takes the 32 rows of one row wavefront, in the partials' register
+// layout (lane l: row l % 32), and of their dims one float4 per lane (F16: 8
+// consecutive dims of a row) or D / 32 (F32: as many consecutive dims per lane
+// and element).  8 parts (F32: 4), weights and rows, are in flight at once: the
+// kernel is bound by its dependent round trips (lengths, then the parts).
+template <int D, bool kF32>
+constexpr int merge_waves_per_tile() {
+  return kRowWaves * (kF32 ? 4 : D / 8);
+}
+template <int D, typename T, int G>
+__global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(PrefillParams p) {
+  constexpr int TT = prefill_tile_tokens<D, T>();
+  constexpr bool kF32 = sizeof(T) == 4;
+  constexpr int kVecs = kF32 ? D / 32 : 1; // float4 per lane
+  constexpr int kBatch = kF32 ? 4 : 8;     // parts in flight
+  constexpr int kPerTile = merge_waves_per_tile<D, kF32>();
+  static_assert(kPerTile % kMergeWaves == 0, "whole blocks per tile");
+  const CallParts<TT, G> call(p);
+  PartPos t;
+  if (!call.split() || !call.template find<Find::kTile>(p, blockIdx.x / (kPerTile / kMergeWaves), t)) return;
+  const int own = (block_key_tiles<TT>(t.s, p.group_size, t.rt) + G - 1) / G; // steps its rows see
+  const int parts = min(t.parts, own);
+  if (parts <= 1) return;
+  const int rts = seq_row_tiles(p, t.s);
   const int l = threadIdx.x & 63;
-  const int ld = kDimLanes == 64 ? l : min(l, kDimLanes - 1); // lane's slice of the row
-  const int rt = tile % p.row_tiles;
-  const int h = (tile / p.row_tiles) % p.num_kv_heads;
-  const int b = p.seq_lo + tile / (p.row_tiles * p.num_kv_heads);
-  const int splits = min(p.kv_splits, kMaxSplits);
-  const int64_t prow0 = (int64_t)tile * p.kv_splits * kBlockRows + lr0; // split j, row r: prow0 + j * kBlockRows + r
-  float mj_raw[kMergeRows], lj_raw[kMergeRows], v[kMergeRows][kMaxSplits][kPer];
+  const int hh = l >> 5;
+  const int unit = blockIdx.x % (kPerTile / kMergeWaves) * kMergeWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rw = unit % kRowWaves, k = unit / kRowWaves; // k: n * 4 + e / 4 (F16) or e / 4 (F32)
+  const int rho = t.rt * kBlockRows + rw * kRowsPerWave + (l & 31);
+  const bool valid = rho < p.group_size * t.s.q_len;
+  const float2v* ml = reinterpret_cast<const float2v*>(p.partial_ml) + (int64_t)t.slot0 * kBlockRows + rw * kRowsPerWave + (l & 31);
+  const float4v* src = reinterpret_cast<const float4v*>(p.partial_o) +
+                       ((int64_t)t.slot0 * kRowWaves + rw) * (D / 8 * 64) + k * 64 + l;
+  float m = -INFINITY, den = 0.f;
+  float4v acc[kVecs];
 #pragma unroll
-  for (int r = 0; r < kMergeRows; r++) {
-    const int64_t pr = prow0 + (int64_t)l * kBlockRows + r;
-    mj_raw[r] = l < splits ? p.partial_ml[pr * 2] : -INFINITY;
-    lj_raw[r] = l < splits ? p.partial_ml[pr * 2 + 1] : 0.f;
+  for (int v = 0; v < kVecs; v++) acc[v] = float4v{0.f, 0.f, 0.f, 0.f};
+  for (int j0 = 0; j0 < parts; j0 += kBatch) {
+    // (Past the last part: its rows again, at weight 0.)
+    float2v mlj[kBatch];
+    float4v o[kBatch][kVecs];
 #pragma unroll
-    for (int j = 0; j < kMaxSplits; j++) {
-      const float* src = p.partial_o + (prow0 + (int64_t)j * kBlockRows + r) * D + ld * kPer;
+    for (int u = 0; u < kBatch; u++) {
+      const int64_t j = min(j0 + u, parts - 1) * rts;
+      mlj[u] = ml[j * kBlockRows];
 #pragma unroll
-      for (int e = 0; e < kPer; e++) v[r][j][e] = j < splits ? src[e] : 0.f;
+      for (int v = 0; v < kVecs; v++) o[u][v] = src[j * kRowWaves * (D / 8 * 64) + 4 * v * 64];
     }
+    float m_new = m;
+#pragma unroll
+    for (int u = 0; u < kBatch; u++) m_new = fmaxf(m_new, mlj[u][0]);
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f(m - m_use); // 0 in the first batch
+    den *= alpha;
+#pragma unroll
+    for (int v = 0; v < kVecs; v++) acc[v] *= alpha;
+#pragma unroll
+    for (int u = 0; u < kBatch; u++) {
+      const float w = j0 + u < parts ? __builtin_amdgcn_exp2f(mlj[u][0] - m_use) : 0.f; // m = -inf (no visible key): 0
+      den += w * mlj[u][1];
+#pragma unroll
+      for (int v = 0; v < kVecs; v++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) acc[v][c] = w == 0.f ? acc[v][c] : fmaf(w, o[u][v][c], acc[v][c]);
+    }
+    m = m_new;
   }
-  const SeqRows s = load_rows(p, b);
-  const int rows = p.group_size * s.q_len;
-  const int n_tiles = block_key_tiles<TT>(s, p.group_size, rt);
-  if (n_tiles == 0) return;
-  const int tiles_per_split = (n_tiles + p.kv_splits - 1) / p.kv_splits;
-  const int n_parts = min((n_tiles + tiles_per_split - 1) / tiles_per_split, splits); // splits that ran
+  if (!valid) return;
+  const int r = rho / t.s.q_len, i = rho % t.s.q_len;
+  const float inv = 1.f / den;
+  const int64_t srow = (int64_t)(t.h * p.group_size + r) * p.state_tokens + t.s.q_start + i;
+  const int64_t orow = (int64_t)(t.h * p.group_size + r) * p.out_stride_head + (int64_t)(t.s.q_start + i) * p.out_stride_token;
+  if (p.state_o && k == 0 && hh == 0) p.state_lse[srow] = (m == -INFINITY ? 0.f : m) + __log2f(den);
+  if constexpr (kF32) {
+    float* dst = (p.state_o ? p.state_o + srow * D : static_cast<float*>(p.out) + orow) + (D / 32) * (8 * k + 4 * hh);
 #pragma unroll
-  for (int r = 0; r < kMergeRows; r++) {
-    const int rho = rt * kBlockRows + lr0 + r;
-    if (rho >= rows) break;
-    const float mj = l < n_parts ? mj_raw[r] : -INFINITY;
-    float mmax = mj;
+    for (int c = 0; c < 4; c++)
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) mmax = fmaxf(mmax, __shfl_xor(mmax, off));
-    const float m_use = mmax == -INFINITY ? 0.f : mmax;
-    const float w = mj == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mj - m_use);
-    float den = l < n_parts ? w * lj_raw[r] : 0.f;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) den += __shfl_xor(den, off);
-    float acc[kPer];
-#pragma unroll
-    for (int e = 0; e < kPer; e++) acc[e] = 0.f;
-#pragma unroll
-    for (int j = 0; j < kMaxSplits; j++) {
-      if (j < n_parts) {
-        const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
-#pragma unroll
-        for (int e = 0; e < kPer; e++) acc[e] = fmaf(wj, v[r][j][e], acc[e]);
-      }
-    }
-    const int qr = rho / s.q_len, i = rho % s.q_len;
-    const float inv = 1.f / den;
-    if (p.state_o) {
-      const int64_t srow = (int64_t)(h * p.group_size + qr) * p.state_tokens + s.q_start + i;
-      if (kDimLanes == 64 || l < kDimLanes) {
-#pragma unroll
-        for (int e = 0; e < kPer; e++) p.state_o[srow * D + ld * kPer + e] = acc[e] * inv;
-      }
-      if (l == 0) p.state_lse[srow] = m_use + __log2f(den);
-      continue;
-    }
-    if (kDimLanes < 64 && l >= kDimLanes) continue;
-    T* dst = static_cast<T*>(p.out) + (int64_t)(h * p.group_size + qr) * p.out_stride_head +
-             (int64_t)(s.q_start + i) * p.out_stride_token + ld * kPer;
-#pragma unroll
-    for (int e = 0; e < kPer; e++) dst[e] = (T)(acc[e] * inv);
+      for (int v = 0; v < kVecs; v++) dst[(D / 32) * c + v] = acc[v][c] * inv;
+  } else {
+    const int d = 8 * k + 4 * hh; // k = 4 n + e / 4: dim 32 n + 8 (e / 4) + 4 hh
+    const float4v o = acc[0] * inv;
+    if (p.state_o)
+      *reinterpret_cast<float4v*>(p.state_o + srow * D + d) = o;
+    else
+      *reinterpret_cast<half4*>(static_cast<half_t*>(p.out) + orow + d) =
+          half4{(half_t)o[0], (half_t)o[1], (half_t)o[2], (half_t)o[3]};
   }
+}
+
+template <int D, typename T, int G, bool TP>
+hipError_t launch_shape(const PrefillParams& params, hipStream_t stream) {
+  if (params.balanced_blocks > 0) {
+    // (One-group blocks up to D=128 are for grids of many blocks per CU.)
+    if constexpr (G == 1 && D <= 128) {
+      return hipErrorInvalidValue;
+    } else {
+      hipLaunchKernelGGL((paged_prefill_balanced_kernel<D, T, G, TP>), dim3((unsigned)params.balanced_blocks),
+                         dim3(kRowWaves * G * 64), 0, stream, params);
+      const hipError_t err = hipGetLastError();
+      if (err != hipSuccess) return err;
+      hipLaunchKernelGGL((prefill_merge_kernel<D, T, G>),
+                         dim3((unsigned)(params.balanced_tiles * (merge_waves_per_tile<D, sizeof(T) == 4>() / kMergeWaves))),
+                         dim3(64 * kMergeWaves), 0, stream, params);
+    }
+  } else {
+    const int64_t blocks = prefill_main_blocks(params) + params.catch_count;
+    hipLaunchKernelGGL((paged_prefill_kernel<D, T, G, TP>), dim3((unsigned)blocks), dim3(kRowWaves * G * 64), 0,
+                       stream, params);
+  }
+  return hipGetLastError();
 }
 
 template <int D, typename T>
 hipError_t launch_typed(const PrefillParams& params, hipStream_t stream) {
-  constexpr int TT = prefill_tile_tokens<D, T>();
-  const int64_t blocks = prefill_main_blocks(params) + params.catch_count;
+  if (params.groups != 1 && (params.groups != 2 || D > 128)) return hipErrorInvalidValue;
   if (params.page_size % 16 != 0) {
     if (!prefill_token_pages_supported(params.page_size, params.num_kv_heads, D, (int)sizeof(T)))
       return hipErrorInvalidValue;
-    if constexpr (D == 64 || D == 128) {
-      if (params.groups == 1)
-        hipLaunchKernelGGL((paged_prefill_kernel<D, T, 1, true>), dim3((unsigned)blocks), dim3(kRowWaves * 64),
-                           0, stream, params);
-      else if (params.groups == 2)
-        hipLaunchKernelGGL((paged_prefill_kernel<D, T, 2, true>), dim3((unsigned)blocks),
-                           dim3(kRowWaves * 2 * 64), 0, stream, params);
-      else
-        return hipErrorInvalidValue;
-    }
-  } else if constexpr (D > 128) {
-    if (params.groups != 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((paged_prefill_kernel<D, T, 1, false>), dim3((unsigned)blocks), dim3(kRowWaves * 64), 0, stream, params);
-  } else if (params.groups == 1) {
-    hipLaunchKernelGGL((paged_prefill_kernel<D, T, 1, false>), dim3((unsigned)blocks), dim3(kRowWaves * 64), 0, stream, params);
-  } else if (params.groups == 2) {
-    hipLaunchKernelGGL((paged_prefill_kernel<D, T, 2, false>), dim3((unsigned)blocks), dim3(kRowWaves * 2 * 64), 0, stream,
-                       params);
-  } else {
+    if constexpr (D == 64 || D == 128)
+      return params.groups == 1 ? launch_shape<D, T, 1, true>(params, stream) : launch_shape<D, T, 2, true>(params, stream);
     return hipErrorInvalidValue;
   }
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess || params.kv_splits == 1) return err;
-  const int64_t split_pairs = (int64_t)(params.seq_count ? params.seq_count : params.num_seqs) * params.num_kv_heads;
-  hipLaunchKernelGGL((prefill_merge_kernel<D, T, TT>),
-                     dim3((unsigned)(split_pairs * params.row_tiles * (kBlockRows / (kMergeWaves * merge_rows<D>())))),
-                     dim3(256), 0, stream, params);
-  return hipGetLastError();
+  if constexpr (D <= 128) {
+    if (params.groups == 2) return launch_shape<D, T, 2, false>(params, stream);
+  }
+  return launch_shape<D, T, 1, false>(params, stream);
 }
 
 } // namespace
