@@ -290,8 +290,7 @@ void plan_balanced(const mvr_paged_attention_args* a, const LiveSeqs& live, int6
 mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_prefill = true,
                                   LiveSeqs live = LiveSeqs{}, bool force_prefill = false) {
   mvr::PagedAttentionPlan plan{};
-  // Sizing inputs (the grid itself always covers num_seqs sequences and the
-  // call's max_seq_len, which the kernels clamp device lengths to).
+  // Sizing inputs (the grid itself always covers num_seqs sequences).
   const int64_t n_live = live.count > 0 && live.count < a->num_seqs ? live.count : a->num_seqs;
   const int len_live = live.max_seq_len > 0 && live.max_seq_len < a->max_seq_len ? live.max_seq_len : a->max_seq_len;
   plan.dtype = a->dtype;
@@ -349,8 +348,10 @@ mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_
   plan.row_blocks = rows_max <= 16 || !all_plans ? 1 : 2;
   const int tile_rows = 16 * plan.row_blocks;
   plan.row_tiles = (int)((rows_max + tile_rows - 1) / tile_rows);
-  const int max_chunks = (a->max_seq_len + mvr::kChunkTokens - 1) / mvr::kChunkTokens; // the grid covers these
-  const int live_chunks = (len_live + mvr::kChunkTokens - 1) / mvr::kChunkTokens;      // and sizes for these
+  // The grid and its partial slots are sized for the longest context of the
+  // launch; a longer one in the device tables (a stale hint) is split into as
+  // many longer partitions (tile_parts).
+  const int max_chunks = (len_live + mvr::kChunkTokens - 1) / mvr::kChunkTokens;
   const int64_t base_units = (int64_t)a->num_seqs * a->num_kv_heads * plan.row_tiles;
   const bool ragged = a->sum_seq_lens > 0 && a->sum_seq_lens < (int64_t)len_live * n_live;
   int cpp = chunks_per_partition_override();
@@ -396,13 +397,13 @@ mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_
       // Every sequence planned at max_seq_len: num_seqs * ceil(max_chunks / c) units.
       int64_t parts = units_per_group / n_live;
       if (parts < 1) parts = 1;
-      c = (live_chunks + parts - 1) / parts;
+      c = (max_chunks + parts - 1) / parts;
     }
     // Floor: small batches are bound by each wavefront's serial chain of
     // chunk loads, so they split down to 4 chunks per wavefront (2 for
     // contexts up to 1024 tokens); measured 17.9 -> 12.1 us on one 512-token
     // F32 sequence and 24 -> 14 us on 8 sequences of 128..4096 tokens.
-    const int64_t floor_cpp = live_chunks <= 64 ? 2 : 4;
+    const int64_t floor_cpp = max_chunks <= 64 ? 2 : 4;
     cpp = (int)(c < floor_cpp ? floor_cpp : (c > max_chunks ? max_chunks : c));
     if (ragged) {
       ragged_units_per_group = units_per_group;
@@ -466,7 +467,7 @@ mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_
     dense = est_live * 10 < (int64_t)a->num_seqs * plan.max_parts * 7; // live fraction < 0.7
   }
   plan.dense_parts = dense;
-  if (dense && ragged_units_per_group > 0 && live_chunks > 64) {
+  if (dense && ragged_units_per_group > 0 && max_chunks > 64) {
     // Dense plans split for 120% of the resident slots instead of 80%:
     // in-order dispatch hands the extra units to whichever CU frees first,
     // and the layout has already given up the cross-sequence partition
@@ -665,6 +666,7 @@ int launch_planned(const mvr_paged_attention_args* a, const mvr::PagedAttentionP
   p.num_kv_heads = a->num_kv_heads;
   p.group_size = a->num_q_heads / a->num_kv_heads;
   p.page_size = a->page_size;
+  p.max_rows = (int32_t)std::min<int64_t>((int64_t)p.group_size * a->max_q_len, INT32_MAX);
   p.scale_log2 = scale * 1.4426950408889634f;
   p.key_begin = cp.key_begin;
   p.key_end = cp.key_end;
@@ -1007,9 +1009,17 @@ CascadePlan make_cascade_plan(const mvr_paged_attention_args* a, const mvr_casca
   c.suf = *a;
   c.suf.sum_seq_lens =
       a->sum_seq_lens > 0 && g->sum_prefix_lens > 0 ? a->sum_seq_lens - g->sum_prefix_lens : a->sum_seq_lens;
-  if (c.suf.sum_seq_lens >= (int64_t)a->max_seq_len * a->num_seqs) c.suf.sum_seq_lens = 0;
+  // Where the hints say that every sequence has the longest prefix, the suffix
+  // pass is sized for the longest suffix instead of the longest context: on 64
+  // sequences of 256..2,048 tokens behind 8,192 shared ones its grid otherwise
+  // holds eight units without keys for one with, and longer partitions.
+  LiveSeqs suf_live;
+  if (g->sum_prefix_lens == (int64_t)a->num_seqs * g->max_prefix_len && a->max_seq_len > g->max_prefix_len)
+    suf_live.max_seq_len = a->max_seq_len - g->max_prefix_len;
+  const int64_t suf_len = suf_live.max_seq_len > 0 ? suf_live.max_seq_len : a->max_seq_len;
+  if (c.suf.sum_seq_lens >= suf_len * a->num_seqs) c.suf.sum_seq_lens = 0;
   // The suffix pass starts every sequence at its prefix: split-context kernel.
-  c.suf_plan = make_plan(&c.suf, /*allow_prefill=*/false);
+  c.suf_plan = make_plan(&c.suf, /*allow_prefill=*/false, suf_live);
   const size_t so = (size_t)a->num_q_heads * c.state_tokens * a->head_dim * sizeof(float);
   const size_t sl = (size_t)a->num_q_heads * c.state_tokens * sizeof(float);
   c.off_suf = align_up(c.pre_plan.partial_bytes, 256);

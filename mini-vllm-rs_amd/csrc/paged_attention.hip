@@ -25,6 +25,7 @@
 
 #include <math.h>
 
+#include <algorithm>
 #include <atomic>
 
 namespace mvr {
@@ -63,28 +64,28 @@ struct SeqInfo {
   int seq_len, q_start, q_len, key_begin, key_end;
 };
 
+// The tables' loads go out together, an absent table's from one that is there:
+// one round trip before a unit starts, not one per table.
 __device__ __forceinline__ SeqInfo load_seq(const PagedAttentionParams& p, int b) {
+  const const_i32* any = (const const_i32*)(p.cu_q_lens ? p.cu_q_lens : p.seq_lens ? p.seq_lens : p.block_tables);
+  const int seq_len = *(p.seq_lens ? (const const_i32*)p.seq_lens + b : any);
+  const int q_start = *(p.cu_q_lens ? (const const_i32*)p.cu_q_lens + b : any);
+  const int q_end = *(p.cu_q_lens ? (const const_i32*)p.cu_q_lens + b + 1 : any);
+  int key_begin = 0, key_end = 0; // cascade passes only
+  if (p.key_begin) key_begin = ((const const_i32*)p.key_begin)[b];
+  if (p.key_end) key_end = ((const const_i32*)p.key_end)[b];
   SeqInfo s;
   // single_seq_len is the call's max_seq_len, whose pages the host has checked
   // to fit a block-table row: a larger device seq_len (a broken contract) is
-  // clamped so that no read leaves the row or the planned partitions.
-  s.seq_len = p.seq_lens ? min(p.seq_lens[b], p.single_seq_len) : p.single_seq_len;
-  if (p.cu_q_lens) {
-    s.q_start = p.cu_q_lens[b];
-    s.q_len = p.cu_q_lens[b + 1] - s.q_start;
-  } else {
-    s.q_start = 0;
-    s.q_len = p.single_q_len;
-  }
+  // clamped so that no read leaves the row.
+  s.seq_len = p.seq_lens ? min(seq_len, p.single_seq_len) : p.single_seq_len;
+  s.q_start = p.cu_q_lens ? q_start : 0;
+  s.q_len = p.cu_q_lens ? q_end - q_start : p.single_q_len;
   // Another launch's sequence: no rows here (every unit of it exits at once).
   if (s.q_len < p.class_q_min || (p.class_q_max > 0 && s.q_len > p.class_q_max)) s.q_len = 0;
-  s.key_begin = p.key_begin ? p.key_begin[b] : 0;
-  if (p.key_end) {
-    s.key_end = p.key_end[b];
-    s.seq_len = s.key_end + s.q_len; // every row's causal limit reaches past the prefix
-  } else {
-    s.key_end = s.seq_len;
-  }
+  s.key_begin = key_begin;
+  s.key_end = p.key_end ? key_end : s.seq_len;
+  if (p.key_end) s.seq_len = key_end + s.q_len; // every row's causal limit reaches past the prefix
   return s;
 }
 
@@ -104,20 +105,23 @@ __device__ __forceinline__ int tile_chunks(const SeqInfo& s, int group_size, int
   return last_key < 0 ? 0 : last_key / kChunkTokens + 1;
 }
 
-// Partitions of a row tile: chunks [key_begin/16, n_chunks) in chunks_per_part pieces.
-__device__ __forceinline__ int tile_parts(const SeqInfo& s, int n_chunks, int chunks_per_part) {
+// Partitions of a row tile: its chunks [key_begin/16, n_chunks) in pieces of
+// chunks_per_part, or in max_parts longer ones where the host planned for
+// shorter contexts than the device tables hold.
+__device__ __forceinline__ int tile_parts(const PagedAttentionParams& p, const SeqInfo& s, int n_chunks) {
   const int kb = s.key_begin / kChunkTokens;
-  return n_chunks > kb ? (n_chunks - kb + chunks_per_part - 1) / chunks_per_part : 0;
+  return n_chunks > kb ? min((n_chunks - kb + p.chunks_per_part - 1) / p.chunks_per_part, p.max_parts) : 0;
 }
 
-// Inclusive prefix sum over the 64 lanes of a wavefront.
+// Inclusive prefix sum over the 64 lanes of a wavefront: rows of 16 by shifts,
+// then each row's last lane into the rows after it (DPP, no LDS round trips).
 __device__ __forceinline__ int wave_inclusive_sum(int v) {
-  const int l = lane_id();
-#pragma unroll
-  for (int off = 1; off < kWaveSize; off <<= 1) {
-    const int t = __shfl_up(v, off);
-    if (l >= off) v += t;
-  }
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false); // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false); // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false); // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false); // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false); // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false); // row_bcast:31 into rows 2 and 3
   return v;
 }
 
@@ -132,46 +136,39 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
 // once.  In-order dispatch then hands out the live units like a work queue,
 // longest first within each 64 sequences, spread over all XCDs.
 __device__ __forceinline__ SeqInfo lane_seq(const SeqInfo& s, int src) {
-  return SeqInfo{__shfl(s.seq_len, src), __shfl(s.q_start, src), __shfl(s.q_len, src), __shfl(s.key_begin, src),
-                 __shfl(s.key_end, src)};
+  auto lane = [&](int v) { return __builtin_amdgcn_readlane(v, src); };
+  return SeqInfo{lane(s.seq_len), lane(s.q_start), lane(s.q_len), lane(s.key_begin), lane(s.key_end)};
 }
 
 // Also returns the sequence's SeqInfo (loaded by one lane of the scan), so the
 // unit starts without a second round trip for it.
-__device__ bool dense_unit(const PagedAttentionParams& p, int64_t w, int tile_rows, int& b_out, int& part_out,
-                           SeqInfo& s_out) {
+// (p.num_units bounds the pairs: an index fits 32 bits.)
+__device__ __forceinline__ bool dense_unit(const PagedAttentionParams& p, int w, int tile_rows, int& b_out,
+                                           int& part_out, SeqInfo& s_out) {
   const int l = lane_id();
-  int64_t base = 0;
+  auto lane = [](int v, int src) { return __builtin_amdgcn_readlane(v, src); };
   for (int b0 = 0; b0 < p.num_seqs; b0 += kWaveSize) {
-    const int b = b0 + l;
-    int n = 0;
-    SeqInfo s{0, 0, 0, 0, 0};
-    if (b < p.num_seqs) {
-      s = load_seq(p, b);
-      n = tile_parts(s, tile_chunks(s, p.group_size, 0, tile_rows), p.chunks_per_part);
-    }
+    const SeqInfo s = load_seq(p, min(b0 + l, p.num_seqs - 1));
+    const int n = b0 + l < p.num_seqs ? tile_parts(p, s, tile_chunks(s, p.group_size, 0, tile_rows)) : 0;
     const int full = n > 0 ? n - 1 : 0, last = n > 0 ? 1 : 0;
     const int full_incl = wave_inclusive_sum(full), last_incl = wave_inclusive_sum(last);
-    const int full_total = __shfl(full_incl, kWaveSize - 1), last_total = __shfl(last_incl, kWaveSize - 1);
-    if (w < base + full_total) {
-      const int64_t r = w - base;
-      const uint64_t hit = __ballot(r >= full_incl - full && r < full_incl);
-      const int src = __builtin_ctzll(hit);
+    const int full_total = lane(full_incl, kWaveSize - 1), last_total = lane(last_incl, kWaveSize - 1);
+    if (w < full_total) {
+      const int src = __builtin_ctzll(__ballot(w < full_incl));
       b_out = b0 + src;
-      part_out = (int)(r - __shfl(full_incl - full, src));
+      part_out = w - lane(full_incl - full, src);
       s_out = lane_seq(s, src);
       return true;
     }
-    if (w < base + full_total + last_total) {
-      const int64_t r = w - base - full_total;
-      const uint64_t hit = __ballot(last == 1 && r == last_incl - 1);
-      const int src = __builtin_ctzll(hit);
+    w -= full_total;
+    if (w < last_total) {
+      const int src = __builtin_ctzll(__ballot(w < last_incl));
       b_out = b0 + src;
-      part_out = __shfl(n, src) - 1;
+      part_out = lane(n, src) - 1;
       s_out = lane_seq(s, src);
       return true;
     }
-    base += full_total + last_total;
+    w -= last_total;
   }
   return false;
 }
@@ -460,9 +457,7 @@ __global__ __launch_bounds__(kWaveSize* WPB, (kernel_min_blocks<Tr, NB, DEPTH, W
   } else if constexpr (DENSE) {
     h = (int)(unit % p.num_kv_heads);
     rt = 0;
-    // part >= max_parts only if a seq_len exceeds max_seq_len (a broken
-    // contract): its partial slot would lie in the next tile, so drop it.
-    if (!dense_unit(p, unit / p.num_kv_heads, kTileRows, b, part, s) || part >= p.max_parts) return;
+    if (!dense_unit(p, (int)(unit / p.num_kv_heads), kTileRows, b, part, s)) return;
   } else {
     int64_t rest = unit;
     h = (int)(rest % p.num_kv_heads);
@@ -484,7 +479,7 @@ __global__ __launch_bounds__(kWaveSize* WPB, (kernel_min_blocks<Tr, NB, DEPTH, W
   // remainder: in a ragged batch the full-length units set the critical path
   // while the remainders finish early.  A uniform batch whose context is a
   // multiple of chunks_per_part gets the same boundaries either way.
-  const int n_parts = tile_parts(s, n_chunks, p.chunks_per_part);
+  const int n_parts = tile_parts(p, s, n_chunks);
   const int kb0 = s.key_begin / kChunkTokens;
   const int64_t span = n_chunks > kb0 ? n_chunks - kb0 : 0;
   const int k0 = n_parts > 0 ? kb0 + (int)((int64_t)part * span / n_parts) : kb0;
@@ -776,7 +771,7 @@ __global__ __launch_bounds__(kWaveSize* WPB, (kernel_min_blocks<Tr, NB, DEPTH, W
 // Merge pass over the partitions of every tile that was split:
 //   out = sum_j 2^(m_j - M) o_j / sum_j 2^(m_j - M) l_j,  M = max_j m_j.
 // One wavefront per (b, h, rt, row); a 256-thread block covers 4 rows of one
-// tile.  Lane j holds partition j's weight (64 partitions per round), the
+// tile (blockIdx.y: as many as the call's longest query can fill).  Lane j holds partition j's weight (64 partitions per round), the
 // partial rows are streamed as one coalesced 4*D-byte row per load with the
 // weight broadcast by readlane, eight rows in flight, or (kWide, for plans of
 // more than 64 partitions per tile) 32 while at least 32 remain and eight
@@ -790,7 +785,6 @@ __global__ __launch_bounds__(kWaveSize* WPB, (kernel_min_blocks<Tr, NB, DEPTH, W
 template <typename T, int D, int NB, bool kWide>
 __global__ __launch_bounds__(256) void merge_partitions_kernel(PagedAttentionParams p) {
   constexpr int kTileRows = 16 * NB;
-  constexpr int kBlocksPerTile = kTileRows / kWavesPerBlock;
   // Output elements per lane: D/64 over the wavefront, or, where D is not a
   // multiple of 64, D/32 over lanes 0..31 (the others hold partition weights
   // only: they re-read lane 31's elements and store nothing).
@@ -798,8 +792,8 @@ __global__ __launch_bounds__(256) void merge_partitions_kernel(PagedAttentionPar
   constexpr int kDimLanes = D / kPer;
   constexpr int kInFlight = 8;
   constexpr int kInFlightWide = kWide ? 32 : kInFlight;
-  const int tile = blockIdx.x / kBlocksPerTile;
-  const int lr = (blockIdx.x % kBlocksPerTile) * kWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+  const int tile = blockIdx.x;
+  const int lr = blockIdx.y * kWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
   const int l = lane_id();
   const int ld = kDimLanes == kWaveSize ? l : min(l, kDimLanes - 1); // lane's slice of the row
   const bool stores = kDimLanes == kWaveSize || l < kDimLanes;
@@ -818,8 +812,7 @@ __global__ __launch_bounds__(256) void merge_partitions_kernel(PagedAttentionPar
   const int rho = rt * kTileRows + lr;
   if (rho >= p.group_size * s.q_len) return;
   const int n_chunks = tile_chunks(s, p.group_size, rt, kTileRows);
-  // At most max_parts partials exist per tile (more only if a seq_len exceeds max_seq_len).
-  const int n_parts = min(tile_parts(s, n_chunks, p.chunks_per_part), p.max_parts);
+  const int n_parts = tile_parts(p, s, n_chunks);
   if (n_parts <= 1) return;
 
   // The first kFirst partial rows need only the partition count: they are in
@@ -1043,11 +1036,13 @@ hipError_t launch_typed(const PagedAttentionPlan& plan, const PagedAttentionPara
   }
   if (err != hipSuccess || plan.max_parts <= 1) return err;
   const int64_t tiles = (int64_t)params.num_seqs * params.num_kv_heads * params.row_tiles;
+  const int row_blocks = std::min((params.max_rows + kWavesPerBlock - 1) / kWavesPerBlock, 16 * NB / kWavesPerBlock);
+  const dim3 grid((unsigned)tiles, (unsigned)row_blocks);
   if (plan.max_parts > 64) {
-    hipLaunchKernelGGL((merge_partitions_kernel<typename Tr::elem, D, NB, true>), dim3((unsigned)(tiles * 4 * NB)),
+    hipLaunchKernelGGL((merge_partitions_kernel<typename Tr::elem, D, NB, true>), grid,
                        dim3(kWaveSize * kWavesPerBlock), 0, stream, params);
   } else {
-    hipLaunchKernelGGL((merge_partitions_kernel<typename Tr::elem, D, NB, false>), dim3((unsigned)(tiles * 4 * NB)),
+    hipLaunchKernelGGL((merge_partitions_kernel<typename Tr::elem, D, NB, false>), grid,
                        dim3(kWaveSize * kWavesPerBlock), 0, stream, params);
   }
   return hipGetLastError();

@@ -52,6 +52,7 @@ struct PagedAttentionParams {
   int32_t max_parts;       // partitions per (sequence, kv head, row tile) in the grid
   int32_t row_tiles;       // row tiles per (sequence, kv head)
   int64_t num_units;
+  int32_t max_rows;     // grouped rows of the longest query (group_size * max_q_len)
   float scale_log2; // softmax scale * log2(e)
   // Cascade passes (all optional, null / 0 otherwise):
   const int32_t* key_begin; // per sequence: first key (a multiple of 16); earlier keys belong to the prefix pass
