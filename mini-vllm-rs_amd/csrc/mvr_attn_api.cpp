@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <functional>
 #include <mutex>
 #include <vector>
 
@@ -178,11 +179,12 @@ int device_cus() {
 struct LiveSeqs {
   int64_t count = 0;   // sequences with rows in this launch (0: num_seqs)
   int max_seq_len = 0; // their longest context (0: the call's max_seq_len)
-  // Prefill kernel: valid host tables of the call, whose sequences of at least
-  // q_min new tokens are the launch's (null: count sequences at the bounds).
+  // Valid host tables of the launch's sequences: those of its num_seqs with
+  // q_min..q_max new tokens (null: count sequences at the bounds above), the
+  // first key_begin keys of each left out.
   const int32_t* cu_q_lens = nullptr;
   const int32_t* seq_lens = nullptr;
-  int q_min = 1;
+  int q_min = 1, q_max = INT32_MAX, key_begin = 0;
   // Largest workspace the balanced prefill grid's partials may take.
   size_t prefill_budget = (size_t)48 << 20;
 };
@@ -285,6 +287,48 @@ void plan_balanced(const mvr_paged_attention_args* a, const LiveSeqs& live, int6
   plan.balanced_slots = (int)std::max<int64_t>(plan.balanced_blocks, std::min(cus, slots));
   const size_t prow = (size_t)plan.balanced_slots * mvr::kPrefillBlockRows;
   plan.partial_bytes = align_up(prow * a->head_dim * sizeof(float), 256) + align_up(prow * 2 * sizeof(float), 256);
+}
+
+// Whether a ragged batch of one-tile sequences runs in 8-wavefront blocks, a
+// block per (sequence, KV head), dispatched longest first (ranked_seq): one
+// launch without partials in HBM, in place of the dense or slot == partition
+// plan and its merge.  One such block is resident per CU, so it needs more
+// tiles than CUs, to fill in behind the longest, and a makespan near the
+// average load: estimated as the longest tile, the average load, or the two
+// tiles that a CU takes where the second round begins, whichever is longest.
+// Measured (F16 D=128, 8 KV heads, cold inputs, dense -> this): 64 x U[512,
+// 3584] 103.6 -> 94.2 us, 64 x U[2K,14K] 368 -> 347, 128 x U[512,3584] 205 ->
+// 193, 64 x U[2000,3500] (slot == partition) 158 -> 127, 48 x U[300,6000] (load
+// 79% of the makespan) 121 -> 115, 40 x U[512,3584] (71%) 71 -> 67; F32 64 x
+// U[256,2048] 122 -> 109, F32 D=64 64 x U[512,3584] 107 -> 97; but 32 x
+// U[1K,7K] (65%) 102 -> 112, 63 x U[200,900] and one of 15,000 62 -> 178, 64
+// x U[128,1024] 36.9 -> 38.0, 256 x U[64,512] 78 -> 105, and F16 D=64 (half the
+// bytes per token) 57.0 -> 57.5 and 191 -> 199.  4-wavefront blocks: 102 and
+// 382 us on the first two.
+bool longest_first_pays(const mvr_paged_attention_args* a, const LiveSeqs& live) {
+  if (!live.seq_lens || !live.cu_q_lens) return false;
+  if (a->head_dim * (a->dtype == MVR_DTYPE_F16 ? 2 : 4) < 256) return false;
+  constexpr int kBlockTokens = 128; // a block's cost beside its keys, in tokens
+  const int cus = device_cus();
+  const int per_round = cus / a->num_kv_heads; // sequences whose tiles the CUs hold at once
+  if (per_round < 1 || a->num_seqs <= per_round) return false;
+  std::vector<int> cost;
+  cost.reserve(a->num_seqs);
+  int64_t sum = 0;
+  for (int s = 0; s < a->num_seqs; s++) {
+    const int q = live.cu_q_lens[s + 1] - live.cu_q_lens[s];
+    if (q < live.q_min || q > live.q_max) continue;
+    cost.push_back(std::max(live.seq_lens[s] - live.key_begin, 0) + kBlockTokens);
+    sum += cost.back();
+  }
+  const int64_t n = (int64_t)cost.size();
+  if (n <= per_round || sum < n * (768 + kBlockTokens)) return false;
+  std::nth_element(cost.begin(), cost.begin() + per_round, cost.end(), std::greater<int>());
+  const int next = cost[per_round]; // the (per_round + 1)-th longest
+  const int last = *std::min_element(cost.begin(), cost.begin() + per_round);
+  const int longest = *std::max_element(cost.begin(), cost.begin() + per_round);
+  const double load = (double)sum * a->num_kv_heads / cus;
+  return load >= 0.7 * std::max({(double)longest, load, (double)last + next});
 }
 
 mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_prefill = true,
@@ -437,6 +481,15 @@ mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_
     for (int w = 4; w <= widest && plan.block_waves == 0; w *= 2)
       if (plan.max_parts <= w && 4 * plan.max_parts >= 3 * w) plan.block_waves = w;
   }
+  static const bool dense_enabled = env_bool("MVR_ATTN_DENSE_RAGGED", true);
+  const bool longest_first = block_merge_enabled && dense_enabled && cpp_override_none && ragged &&
+                             plan.row_blocks == 1 && plan.row_tiles == 1 && all_plans && !plan.token_pages &&
+                             longest_first_pays(a, live);
+  if (longest_first) {
+    plan.block_waves = 8; // each tile's chunks split evenly over the block
+    plan.max_parts = 8;
+    plan.chunks_per_part = 1;
+  }
   plan.block_merge = plan.block_waves > 0;
   // Dense layout for ragged batches with one row tile (dense_unit in
   // paged_attention.hip): the live units are numbered from 0, so in-order
@@ -458,8 +511,7 @@ mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_
   // tokens per page (64 ragged sequences of 2,048..14,336 tokens in 8-token
   // pages 468 -> 431 us, the others within 1%); in 5-token pages it lost up
   // to 3.5% on shorter contexts.  MVR_ATTN_DENSE_RAGGED=false turns it off.
-  static const bool dense_enabled = env_bool("MVR_ATTN_DENSE_RAGGED", true);
-  bool dense = false;
+  bool dense = longest_first;
   if (dense_enabled && ragged && plan.row_tiles == 1 && plan.max_parts > 1 && !plan.block_merge && n_live >= 32 &&
       (!plan.token_pages || a->page_size >= 8) && all_plans) {
     const int64_t chunk_tokens = (int64_t)mvr::kChunkTokens * plan.chunks_per_part;
@@ -467,7 +519,7 @@ mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_
     dense = est_live * 10 < (int64_t)a->num_seqs * plan.max_parts * 7; // live fraction < 0.7
   }
   plan.dense_parts = dense;
-  if (dense && ragged_units_per_group > 0 && max_chunks > 64) {
+  if (dense && !longest_first && ragged_units_per_group > 0 && max_chunks > 64) {
     // Dense plans split for 120% of the resident slots instead of 80%:
     // in-order dispatch hands the extra units to whichever CU frees first,
     // and the layout has already given up the cross-sequence partition
@@ -717,11 +769,10 @@ int check_workspace(const mvr_paged_attention_args* a, size_t need) {
 // context splits), and a stale hint costs speed, never rows.
 constexpr int kSmallRows = 32;
 
-// The call's host tables for a prefill launch of the sequences with at least
-// q_min new tokens, if both are there and within the call's bounds.
-void prefill_tables(const mvr_paged_attention_args* a, int q_min, LiveSeqs& live) {
-  const int group = a->num_q_heads / a->num_kv_heads;
-  if (!a->cu_q_lens_host || !a->seq_lens_host || (int64_t)group * a->max_q_len <= 64) return;
+// The call's host tables for a launch of the sequences with q_min..q_max new
+// tokens, if both are there and within the call's bounds.
+void use_tables(const mvr_paged_attention_args* a, int q_min, int q_max, LiveSeqs& live) {
+  if (!a->cu_q_lens_host || !a->seq_lens_host) return;
   for (int s = 0; s < a->num_seqs; s++) {
     const int q = a->cu_q_lens_host[s + 1] - a->cu_q_lens_host[s];
     const int L = a->seq_lens_host[s];
@@ -730,6 +781,7 @@ void prefill_tables(const mvr_paged_attention_args* a, int q_min, LiveSeqs& live
   live.cu_q_lens = a->cu_q_lens_host;
   live.seq_lens = a->seq_lens_host;
   live.q_min = q_min;
+  live.q_max = q_max;
 }
 
 struct CallPlan {
@@ -747,7 +799,7 @@ CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget) {
   c.part[0] = *a;
   LiveSeqs all;
   all.prefill_budget = budget;
-  prefill_tables(a, 1, all);
+  use_tables(a, 1, INT32_MAX, all);
   c.plan[0] = make_plan(a, true, all);
   c.total = c.plan[0].partial_bytes;
   const int group = a->num_q_heads / a->num_kv_heads;
@@ -811,13 +863,16 @@ CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget) {
   p0.block_tables = a->block_tables ? a->block_tables + (int64_t)f * a->max_pages_per_seq : nullptr;
   p0.seq_lens = a->seq_lens ? a->seq_lens + f : nullptr;
   p0.cu_q_lens = a->cu_q_lens ? a->cu_q_lens + f : nullptr; // q_start stays the whole call's packed index
-  p0.seq_lens_host = nullptr;
-  p0.cu_q_lens_host = nullptr;
   p0.max_q_len = qmax;
   LiveSeqs live0;
   live0.count = count[0];
   if (hinted) {
     if (sl) live0.max_seq_len = lmax[0];
+    use_tables(a, 1, qmax, live0);
+    if (live0.seq_lens) {
+      live0.cu_q_lens += f;
+      live0.seq_lens += f;
+    }
     p0.sum_seq_lens = sl ? lsum[0] : 0; // this class's keys (a speed hint)
   }
   c.plan[0] = make_plan(&p0, /*allow_prefill=*/false, live0);
@@ -826,12 +881,10 @@ CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget) {
   // Launch 1: every sequence that launch 0 leaves.
   mvr_paged_attention_args& p1 = c.part[1];
   p1 = *a;
-  p1.seq_lens_host = nullptr;
-  p1.cu_q_lens_host = nullptr;
   LiveSeqs live1;
   live1.count = count[1];
   live1.prefill_budget = budget;
-  if (hinted) prefill_tables(a, qmax + 1, live1);
+  if (hinted) use_tables(a, qmax + 1, INT32_MAX, live1);
   if (hinted) {
     if (sl) live1.max_seq_len = lmax[1];
     p1.sum_seq_lens = sl ? lsum[1] : 0;
@@ -1014,8 +1067,11 @@ CascadePlan make_cascade_plan(const mvr_paged_attention_args* a, const mvr_casca
   // sequences of 256..2,048 tokens behind 8,192 shared ones its grid otherwise
   // holds eight units without keys for one with, and longer partitions.
   LiveSeqs suf_live;
-  if (g->sum_prefix_lens == (int64_t)a->num_seqs * g->max_prefix_len && a->max_seq_len > g->max_prefix_len)
+  if (g->sum_prefix_lens == (int64_t)a->num_seqs * g->max_prefix_len && a->max_seq_len > g->max_prefix_len) {
     suf_live.max_seq_len = a->max_seq_len - g->max_prefix_len;
+    use_tables(a, 1, INT32_MAX, suf_live);
+    suf_live.key_begin = g->max_prefix_len;
+  }
   const int64_t suf_len = suf_live.max_seq_len > 0 ? suf_live.max_seq_len : a->max_seq_len;
   if (c.suf.sum_seq_lens >= suf_len * a->num_seqs) c.suf.sum_seq_lens = 0;
   // The suffix pass starts every sequence at its prefix: split-context kernel.

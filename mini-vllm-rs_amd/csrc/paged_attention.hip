@@ -173,6 +173,28 @@ __device__ __forceinline__ bool dense_unit(const PagedAttentionParams& p, int w,
   return false;
 }
 
+// Longest first: the sequence of rank `rank` when a batch's sequences are
+// dispatched in decreasing order of their chunks.  The sequences are dealt to
+// ceil(num_seqs / 64) strided groups, whose members (one per lane) are ranked
+// by counting the longer ones, equal ones in lane order: a bijection whatever
+// the tables hold.
+__device__ __forceinline__ void ranked_seq(const PagedAttentionParams& p, int rank, int tile_rows, int& b_out,
+                                           SeqInfo& s_out) {
+  const int groups = (p.num_seqs + kWaveSize - 1) / kWaveSize;
+  const int first = rank % groups, r = rank / groups;
+  const int l = lane_id();
+  const int b = first + groups * l;
+  const int members = (p.num_seqs - first + groups - 1) / groups;
+  const SeqInfo s = load_seq(p, min(b, p.num_seqs - 1));
+  const int n = l < members ? tile_chunks(s, p.group_size, 0, tile_rows) - s.key_begin / kChunkTokens : 0;
+  const int key = max(n, 0) * kWaveSize + (kWaveSize - 1 - l); // distinct per lane
+  int longer = 0;
+  for (int j = 0; j < members; j++) longer += __builtin_amdgcn_readlane(key, j) > key ? 1 : 0;
+  const int src = __builtin_ctzll(__ballot(l < members && longer == r));
+  b_out = first + groups * src;
+  s_out = lane_seq(s, src);
+}
+
 // Cascade suffix pass: weights that merge this pass's normalised row (log2
 // sum lb) with the prefix pass's state of the same row (srow):
 //   out = (wa * o_a + wb * o_b) * inv.
@@ -452,8 +474,13 @@ __global__ __launch_bounds__(kWaveSize* WPB, (kernel_min_blocks<Tr, NB, DEPTH, W
     part = wave;
     h = (int)(tile % p.num_kv_heads);
     tile /= p.num_kv_heads;
-    rt = (int)(tile % p.row_tiles);
-    b = (int)(tile / p.row_tiles);
+    if constexpr (DENSE) {
+      rt = 0;
+      ranked_seq(p, (int)tile, kTileRows, b, s);
+    } else {
+      rt = (int)(tile % p.row_tiles);
+      b = (int)(tile / p.row_tiles);
+    }
   } else if constexpr (DENSE) {
     h = (int)(unit % p.num_kv_heads);
     rt = 0;
@@ -470,7 +497,7 @@ __global__ __launch_bounds__(kWaveSize* WPB, (kernel_min_blocks<Tr, NB, DEPTH, W
   // Partials are stored tile-major: slot = tile * max_parts + part.
   const int64_t slot = (((int64_t)b * p.num_kv_heads + h) * p.row_tiles + rt) * p.max_parts + part;
 
-  if constexpr (BM || !DENSE) s = load_seq(p, b);
+  if constexpr (!DENSE) s = load_seq(p, b);
   const int rows = p.group_size * s.q_len;
   const int n_chunks = tile_chunks(s, p.group_size, rt, kTileRows);
   // The tile's n_parts partitions split its chunks evenly (their lengths differ
@@ -996,6 +1023,17 @@ hipError_t launch_typed(const PagedAttentionPlan& plan, const PagedAttentionPara
                              dim3(kWaveSize * 4), 0, stream, params);
         } else if (plan.block_waves == 8) {
           hipLaunchKernelGGL((paged_attention_kernel<Tr, D, NB, true, false, 2, 8, true>), dim3((unsigned)tiles),
+                             dim3(kWaveSize * 8), 0, stream, params);
+        } else {
+          return hipErrorInvalidValue;
+        }
+      } else if (plan.dense_parts) { // longest first
+        if (params.row_tiles != 1) return hipErrorInvalidValue;
+        if (plan.block_waves == 4) {
+          hipLaunchKernelGGL((paged_attention_kernel<Tr, D, NB, true, true, 2, 4>), dim3((unsigned)tiles),
+                             dim3(kWaveSize * 4), 0, stream, params);
+        } else if (plan.block_waves == 8) {
+          hipLaunchKernelGGL((paged_attention_kernel<Tr, D, NB, true, true, 2, 8>), dim3((unsigned)tiles),
                              dim3(kWaveSize * 8), 0, stream, params);
         } else {
           return hipErrorInvalidValue;
