@@ -185,8 +185,7 @@ struct LiveSeqs {
   const int32_t* cu_q_lens = nullptr;
   const int32_t* seq_lens = nullptr;
   int q_min = 1, q_max = INT32_MAX, key_begin = 0;
-  int64_t split_count = 0; // prefill kernel: sequences of the main grid (0: num_seqs)
-  // Largest workspace a split prefill grid's partials may take.
+  // Largest workspace the balanced prefill grid's partials may take.
   size_t prefill_budget = (size_t)48 << 20;
 };
 
@@ -196,22 +195,20 @@ int prefill_step_keys(const mvr_paged_attention_args* a) {
   return (a->dtype == MVR_DTYPE_F16 ? 64 : 32) * (a->head_dim > 128 ? 1 : 2);
 }
 
-// Split prefill grids (each row tile's keys in parts of at most part_steps
+// Balanced prefill grid (each row tile's keys in parts of at most part_steps
 // steps, a block per part, and a merge launch) where the unsplit one, a block
 // per row tile, leaves CUs idle or waits for its longest sequence.
 // For one to four rounds of blocks over the CUs, and for fewer parts that leave
 // CUs idle: the shortest parts whose blocks fit, and their estimated time.
-// Measured (one box, HIP events): a step of the two-group block at D=128 takes
+// Measured at D=128 (one box, HIP events): a step of the two-group block takes
 // 1.5 us in F16 and 6.9 us in F32 alone and 0.5 / 0.9 us more with every CU
-// busy (F16 at D=64 0.63 of that: its softmax does not shrink); a block costs
-// 8 us beside its steps; splitting costs 3 us (a launch), up to 3 more for the
-// merge of 64 tiles and 3.5 for a CU-full of partial rows.  F16, 256 tokens on
-// 2,048, 64 tiles: 36.1 us unsplit, 33.1 / 29.1 / 28.5 in 2 / 3 / 4 parts; 100
-// on 7,544, 24 tiles: 96.6, and 49.0 / 41.4 / 33.6 / 31.4 in 3 / 4 / 6 / 8; D=64,
-// 70 on 1,049, 8 tiles: 16.1, and 14.7 / 13.2 in 4 / 6; 2 x 153 on 600, 72
-// tiles: 18.5, 22.9 in 2; F32, 3 x 217 on 897..2,320: 309 unsplit, 168 in parts
-// of at most 20 steps.
-void plan_prefill_splits(const mvr_paged_attention_args* a, const LiveSeqs& live, int64_t n_live, int len_live,
+// busy; a block costs 8 us beside its steps; a split call 5 us for the merge
+// and 11 us per CU-full of parts for their partial rows (64 KiB each, written
+// and read) and their cold start.  F16, 256 tokens on 2,048, 64 tiles: 37.0 us
+// unsplit, 36.1 / 33.7 / 36.0 in 2 / 3 / 4 parts; 64 on 8,128, 16 tiles: 102.7,
+// and 51.5 / 41.4 / 33.7 / 29.7 in 3 / 4 / 6 / 8; F32, 3 x 217 tokens on
+// 897..2,320: 309 unsplit, 168 in parts of at most 20 steps.
+void plan_balanced(const mvr_paged_attention_args* a, const LiveSeqs& live, int64_t n_live, int len_live,
                    mvr::PagedAttentionPlan& plan) {
   const int64_t cus = device_cus();
   const int group = a->num_q_heads / a->num_kv_heads;
@@ -230,9 +227,7 @@ void plan_prefill_splits(const mvr_paged_attention_args* a, const LiveSeqs& live
     }
   };
   int64_t tiles = 0, steps = 0, longest = 0;
-  bool equal = true;
   each([&](int64_t t, int64_t n) {
-    equal = equal && (tiles == 0 || n == longest);
     tiles += t;
     steps += t * n;
     longest = std::max(longest, n);
@@ -255,12 +250,10 @@ void plan_prefill_splits(const mvr_paged_attention_args* a, const LiveSeqs& live
   static const int split_override = env_int("MVR_ATTN_PREFILL_SPLITS", 0);
   auto cost_us = [&](int64_t blocks, int64_t part) {
     const double fill = std::min(1.0, (double)blocks / cus);
-    const double step = f16 ? (1.5 + 0.5 * fill) * (0.25 + 0.75 * a->head_dim / 128)
-                            : (6.9 + 0.9 * fill) * a->head_dim / 128;
+    const double step = ((f16 ? 1.5 : 6.9) + (f16 ? 0.5 : 0.9) * fill) * a->head_dim / 128;
     const double load = blocks <= cus ? (double)part : std::max((double)part, (double)steps / cus + part / 2);
     return load * step + 8.0 * ((blocks + cus - 1) / cus);
   };
-  auto split_us = [&](int64_t blocks) { return 3 + 3 * std::min(1.0, tiles / 64.0) + 3.5 * blocks / cus; };
   double best = split_override > 1 ? INFINITY : 0.97 * cost_us(tiles, longest);
   int64_t best_part = 0;
   for (int64_t quarters : {1, 2, 3, 4, 8, 12, 16}) { // of a block per CU
@@ -277,45 +270,22 @@ void plan_prefill_splits(const mvr_paged_attention_args* a, const LiveSeqs& live
     if (lo >= longest) continue;
     int64_t part = 0;
     const int64_t blocks = blocks_at(lo, &part);
-    // (The look-ups of an unequal call's blocks and merge: about 3 us.)
-    const double cost = cost_us(blocks, part) + split_us(blocks) + (equal ? 0 : 3);
+    const double cost = cost_us(blocks, part) + 5 + 11.0 * blocks / cus * a->head_dim / 128;
     if (cost < best) {
       best = cost;
       best_part = lo;
     }
     if (split_override > 1) break;
   }
-  // The main grid with every tile in as many parts (no look-ups: 24 + 7 against
-  // 26 + 9 us on 256 F16 tokens on 2,048) for sequences of one length, and for
-  // others where it is estimated to be no slower.
-  const int64_t span = live.split_count > 0 && live.split_count < a->num_seqs ? live.split_count : a->num_seqs;
-  const int64_t span_tiles = span * a->num_kv_heads * plan.row_tiles;
-  int64_t splits = equal && best_part > 0 ? std::min<int64_t>((longest + best_part - 1) / best_part, mvr::kPrefillMaxParts) : 1;
-  if (!equal && split_override == 0)
-    for (int64_t k = 2; k <= 8 && tiles * k <= cus && 2 * k <= longest; k++) {
-      const double cost = cost_us(tiles * k, (longest + k - 1) / k) + split_us(tiles * k);
-      if (cost <= best) {
-        best = cost;
-        splits = k;
-      }
-    }
-  int64_t used;
-  if (splits > 1 && span_tiles * splits <= slots) {
-    plan.kv_splits = (int)splits;
-    used = span_tiles * splits;
-  } else {
-    // (Part counts are 32-bit on the device, whatever its tables hold.)
-    if (best_part == 0 || (int64_t)a->num_seqs * a->num_kv_heads * plan.row_tiles * mvr::kPrefillMaxParts >= (1LL << 31))
-      return;
-    plan.part_steps = (int)best_part;
-    plan.balanced_blocks = (int)blocks_at(best_part);
-    plan.balanced_tiles = (int)tiles;
-    used = plan.balanced_blocks;
-  }
+  // (Part counts are 32-bit on the device, whatever its tables hold.)
+  if (best_part == 0 || (int64_t)a->num_seqs * a->num_kv_heads * plan.row_tiles * mvr::kPrefillMaxParts >= (1LL << 31)) return;
+  plan.part_steps = (int)best_part;
+  plan.balanced_blocks = (int)blocks_at(best_part);
+  plan.balanced_tiles = (int)tiles;
   // Slots for a block per CU at least: up to there the workspace does not
   // depend on the lengths.
-  plan.partial_slots = (int)std::max(used, std::min(cus, slots));
-  const size_t prow = (size_t)plan.partial_slots * mvr::kPrefillBlockRows;
+  plan.balanced_slots = (int)std::max<int64_t>(plan.balanced_blocks, std::min(cus, slots));
+  const size_t prow = (size_t)plan.balanced_slots * mvr::kPrefillBlockRows;
   plan.partial_bytes = align_up(prow * a->head_dim * sizeof(float), 256) + align_up(prow * 2 * sizeof(float), 256);
 }
 
@@ -416,8 +386,7 @@ mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_
       plan.prefill_groups = groups_override;
     else
       plan.prefill_groups = a->dtype == MVR_DTYPE_F16 && live_blocks >= 4LL * device_cus() ? 1 : 2;
-    plan.kv_splits = 1;
-    if (plan.prefill_groups == 2 || a->head_dim > 128) plan_prefill_splits(a, live, n_live, len_live, plan);
+    if (plan.prefill_groups == 2 || a->head_dim > 128) plan_balanced(a, live, n_live, len_live, plan);
     return plan;
   }
   plan.row_blocks = rows_max <= 16 || !all_plans ? 1 : 2;
@@ -688,7 +657,7 @@ int launch_planned(const mvr_paged_attention_args* a, const mvr::PagedAttentionP
     f.out_stride_head = a->out_stride_head;
     f.out_stride_token = a->out_stride_token;
     if (plan.partial_bytes) {
-      const size_t prow = (size_t)plan.partial_slots * mvr::kPrefillBlockRows;
+      const size_t prow = (size_t)plan.balanced_slots * mvr::kPrefillBlockRows;
       char* w = static_cast<char*>(ws);
       f.partial_o = reinterpret_cast<float*>(w);
       f.partial_ml = reinterpret_cast<float*>(w + align_up(prow * a->head_dim * sizeof(float), 256));
@@ -699,7 +668,6 @@ int launch_planned(const mvr_paged_attention_args* a, const mvr::PagedAttentionP
     f.page_size = a->page_size;
     mvr::page_divider(a->page_size, f.page_magic, f.page_magic_shift);
     f.row_tiles = plan.row_tiles;
-    f.kv_splits = plan.kv_splits;
     f.balanced_blocks = plan.balanced_blocks;
     f.part_steps = plan.part_steps;
     f.balanced_tiles = plan.balanced_tiles;
@@ -915,7 +883,6 @@ CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget) {
   p1 = *a;
   LiveSeqs live1;
   live1.count = count[1];
-  live1.split_count = last[1] - first[1] + 1;
   live1.prefill_budget = budget;
   if (hinted) use_tables(a, qmax + 1, INT32_MAX, live1);
   if (hinted) {

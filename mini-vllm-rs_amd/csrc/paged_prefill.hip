@@ -886,105 +886,105 @@ struct PartPos {
   int b, h, rt, part, parts, slot0; // slot0: the slot of the tile's part 0; part j's is slot0 + j * row tiles
 };
 
-// Row tiles of a sequence over all KV heads, and parts per tile.
+// 64 sequences from b0 on, one per lane: the parts of each, their inclusive
+// sum and total (nothing past the last sequence or for another launch's).
 template <int TT, int G>
-__device__ __forceinline__ void seq_parts(const PrefillParams& p, const SeqRows& s, bool split, int& tiles,
-                                          int& per_tile) {
-  tiles = s.q_len > 0 && s.key_end > 0 ? p.num_kv_heads * seq_row_tiles(p, s) : 0;
-  const unsigned steps = (unsigned)(max(s.key_end, 0) + G * TT - 1) / (G * TT);
-  per_tile = split ? min((int)((steps + p.part_steps - 1) / (unsigned)p.part_steps), kMaxParts) : 1;
-}
-
-// Part (or tile) `rel` of w.s, whose parts start at slot `slot`.
-template <Find kFind>
-__device__ __forceinline__ void place(const PrefillParams& p, int rel, int slot, PartPos& w) {
-  const int rts = seq_row_tiles(p, w.s);
-  if (kFind == Find::kPart) {
-    w.h = (unsigned)rel / (unsigned)(w.parts * rts);
-    const int in_head = rel - w.h * w.parts * rts;
-    w.part = (unsigned)in_head / (unsigned)rts;
-    w.rt = in_head - w.part * rts;
-  } else {
-    w.h = (unsigned)rel / (unsigned)rts;
-    w.part = 0;
-    w.rt = rel - w.h * rts;
+struct SeqParts {
+  SeqRows s;
+  int per_tile, tiles, incl, total, tiles_incl;
+  __device__ __forceinline__ SeqParts(const PrefillParams& p, int b0, bool split) : per_tile(0), tiles(0) {
+    const int b = b0 + (int)(threadIdx.x & 63);
+    s = load_lane_rows(p, min(b, p.num_seqs - 1));
+    if (b < p.num_seqs && s.q_len > 0 && s.key_end > 0) {
+      tiles = p.num_kv_heads * seq_row_tiles(p, s);
+      const int steps = (s.key_end + G * TT - 1) / (G * TT);
+      per_tile = split ? min((int)((unsigned)(steps + p.part_steps - 1) / (unsigned)p.part_steps), kMaxParts) : 1;
+    }
+    incl = wave_inclusive_sum(per_tile * tiles);
+    total = __builtin_amdgcn_readlane(incl, 63);
+    tiles_incl = wave_inclusive_sum(tiles);
   }
-  w.slot0 = slot + w.h * w.parts * rts + w.rt;
-}
+};
 
-// Part i of the call, or (kTile) part 0 of its tile i; false past the last
-// one.  `split`: whether the call is split at all.  The sequences are scanned
-// 64 at a time, one per lane.  (Up to 8 sequences walked with scalar loads
-// instead: 189 against 182 us on three ragged F32 chunks.)
-template <Find kFind, int TT, int G>
-__device__ __forceinline__ bool find_part(const PrefillParams& p, int i, PartPos& w, bool& split) {
-  split = true;
-  auto lane = [](int v, int src) { return __builtin_amdgcn_readlane(v, src); };
-  for (;;) {
-    int left = i, rel = -1, slot0 = 0, slots = 0, all_tiles = 0;
+// The call's parts; the first 64 sequences' stay in registers.
+template <int TT, int G>
+class CallParts {
+  bool split_;
+  SeqParts<TT, G> head_;
+  int total_, tiles_;
+  __device__ __forceinline__ void sum(const PrefillParams& p) {
+    total_ = head_.total;
+    tiles_ = lane(head_.tiles_incl, 63);
+    for (int b0 = 64; b0 < p.num_seqs; b0 += 64) {
+      const SeqParts<TT, G> c(p, b0, split_);
+      total_ += c.total;
+      tiles_ += lane(c.tiles_incl, 63);
+    }
+  }
+  __device__ __forceinline__ static int lane(int v, int src) { return __builtin_amdgcn_readlane(v, src); }
+
+ public:
+  __device__ __forceinline__ explicit CallParts(const PrefillParams& p) : split_(true), head_(p, 0, true) {
+    sum(p);
+    if (total_ > p.balanced_blocks || tiles_ > p.balanced_tiles) {
+      split_ = false;
+      head_ = SeqParts<TT, G>(p, 0, false);
+      sum(p);
+    }
+  }
+  __device__ __forceinline__ bool split() const { return split_; }
+  // Part i, or (kTile) part 0 of tile i; false past the last one.
+  template <Find kFind>
+  __device__ __forceinline__ bool find(const PrefillParams& p, int i, PartPos& w) const {
+    int slot = 0;
     for (int b0 = 0; b0 < p.num_seqs; b0 += 64) {
-      const int b = b0 + (int)(threadIdx.x & 63);
-      const SeqRows s = load_lane_rows(p, min(b, p.num_seqs - 1));
-      int tiles, per_tile;
-      seq_parts<TT, G>(p, s, split, tiles, per_tile);
-      if (b >= p.num_seqs) tiles = 0;
-      const int parts_incl = wave_inclusive_sum(per_tile * tiles), tiles_incl = wave_inclusive_sum(tiles);
-      const int incl = kFind == Find::kPart ? parts_incl : tiles_incl;
+      const SeqParts<TT, G> c = b0 == 0 ? head_ : SeqParts<TT, G>(p, b0, split_);
+      const int incl = kFind == Find::kPart ? c.incl : c.tiles_incl;
+      const int n = kFind == Find::kPart ? c.per_tile * c.tiles : c.tiles;
       const int total = lane(incl, 63);
-      if (rel < 0 && left < total) {
-        const int src = __builtin_ctzll(__ballot(left < incl));
-        w.s = SeqRows{lane(s.seq_len, src), lane(s.q_start, src), lane(s.q_len, src), lane(s.key_end, src)};
+      if (i < total) {
+        const int src = __builtin_ctzll(__ballot(i < incl));
+        const int rel = i - lane(incl - n, src);
+        w.s = SeqRows{lane(c.s.seq_len, src), lane(c.s.q_start, src), lane(c.s.q_len, src), lane(c.s.key_end, src)};
         w.b = b0 + src;
-        w.parts = lane(per_tile, src);
-        rel = left - lane(incl - (kFind == Find::kPart ? per_tile * tiles : tiles), src);
-        slot0 = slots + lane(parts_incl - per_tile * tiles, src);
+        w.parts = lane(c.per_tile, src);
+        const int rts = seq_row_tiles(p, w.s);
+        if (kFind == Find::kPart) {
+          w.h = (unsigned)rel / (unsigned)(w.parts * rts);
+          const int in_head = rel - w.h * w.parts * rts;
+          w.part = (unsigned)in_head / (unsigned)rts;
+          w.rt = in_head - w.part * rts;
+        } else {
+          w.h = (unsigned)rel / (unsigned)rts;
+          w.part = 0;
+          w.rt = rel - w.h * rts;
+        }
+        w.slot0 = slot + lane(c.incl - c.per_tile * c.tiles, src) + w.h * w.parts * rts + w.rt;
+        return true;
       }
-      left -= total;
-      slots += lane(parts_incl, 63);
-      all_tiles += lane(tiles_incl, 63);
+      i -= total;
+      slot += c.total;
     }
-    if (split && (slots > p.balanced_blocks || all_tiles > p.balanced_tiles)) {
-      split = false;
-      continue;
-    }
-    if (rel < 0) return false;
-    place<kFind>(p, rel, slot0, w);
-    return true;
+    return false;
   }
-}
+};
 
-// Main grid: block x covers (sequence, kv head, row tile, part) of the main
-// range, every tile in kv_splits parts (1: unsplit).  XCD-aware decode: block x runs on XCD x % 8 and all blocks of one
+// Main grid: block x covers (sequence, kv head, row tile) of the main range,
+// unsplit.  XCD-aware decode: block x runs on XCD x % 8 and all blocks of one
 // (sequence, kv head) pair sit on the same XCD, so their shared K/V stays in
 // that XCD's L2 (with fewer pairs than XCDs, plain linear order keeps every
 // XCD busy).  Catch-up blocks follow the main grid.
 __host__ __device__ __forceinline__ int64_t prefill_main_blocks(const PrefillParams& p) {
   const int64_t pairs = (int64_t)(p.seq_count ? p.seq_count : p.num_seqs) * p.num_kv_heads;
-  const int64_t per_pair = (int64_t)p.row_tiles * p.kv_splits;
+  const int64_t per_pair = p.row_tiles;
   return pairs >= kXcds ? kXcds * ((pairs + kXcds - 1) / kXcds) * per_pair : pairs * per_pair;
 }
 
 constexpr int kAllSteps = 1 << 24; // past every tile's last step
 
-// Steps of part `part` of a tile in `parts` parts: an even share of the steps
-// that its rows see (fewer parts than that many hold any).
-struct PartSteps {
-  int begin, end, parts; // parts that hold steps
-};
-template <int TT, int G>
-__device__ __forceinline__ PartSteps part_steps(const PrefillParams& p, const SeqRows& s, int rt, int parts, int part) {
-  const int own = (block_key_tiles<TT>(s, p.group_size, rt) + G - 1) / G;
-  const int k = min(parts, own);
-  if (part >= k) return {0, 0, k};
-  const int each = (unsigned)own / (unsigned)k, rest = own - each * k; // the first `rest` parts take one more
-  return {part * each + min(part, rest), (part + 1) * each + min(part + 1, rest), k};
-}
-
 // TP: pages that are not a multiple of 16 tokens, read in place (head_dim 64
-// and 128; the page size a multiple of the tokens one load covers).  SPLIT:
-// kv_splits > 1 (apart, so that an unsplit block starts without its arithmetic:
-// 0.6 of 8.4 us on a small chunk).
-template <int D, typename T, int G, bool TP, bool SPLIT>
+// and 128; the page size a multiple of the tokens one load covers).
+template <int D, typename T, int G, bool TP>
 __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) void paged_prefill_kernel(PrefillParams p) {
   constexpr int TT = prefill_tile_tokens<D, T>();
   const int x = blockIdx.x;
@@ -1003,7 +1003,7 @@ __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) vo
       }
     return;
   }
-  const int per_pair = SPLIT ? p.row_tiles * p.kv_splits : p.row_tiles;
+  const int per_pair = p.row_tiles;
   const int pairs = main_seqs * p.num_kv_heads;
   int pair, local;
   if (pairs >= kXcds) {
@@ -1029,26 +1029,16 @@ __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) vo
   // fresh prompts: Llama-3-8B 1 x 2048 F16 75.3 (in order) -> 70.7 (reverse)
   // -> 58.0 us (by position), F32 512.1 -> 480.6 -> 325.9, Qwen2-7B 1 x 8192
   // 667.7 -> 632.6 -> 517.4; chunks on a long prefix level.
-  int rt, part;
+  int rt;
   {
-    const int idx = SPLIT ? (int)((unsigned)local / (unsigned)p.kv_splits) : local;
-    part = SPLIT ? local - idx * p.kv_splits : 0;
     const int tq = s.q_len / kBlockRows; // tiles per query head
     if (s.q_len > 0 && s.q_len % kBlockRows == 0) {
-      rt = idx < p.group_size * tq ? (idx % p.group_size) * tq + (tq - 1 - idx / p.group_size) : idx;
+      rt = local < p.group_size * tq ? (local % p.group_size) * tq + (tq - 1 - local / p.group_size) : local;
     } else {
-      rt = p.row_tiles - 1 - idx;
+      rt = p.row_tiles - 1 - local;
     }
   }
-  int step0 = 0, step1 = kAllSteps, slot = 0;
-  if constexpr (SPLIT) {
-    const PartSteps steps = part_steps<TT, G>(p, s, rt, p.kv_splits, part);
-    if (steps.begin >= steps.end) return;
-    step0 = steps.begin;
-    step1 = steps.end;
-    slot = (((b - p.seq_lo) * p.num_kv_heads + h) * p.row_tiles + rt) * p.kv_splits + part;
-  }
-  prefill_tile_serial<D, T, TT, G, TP>(p, s, b, h, rt, step0, step1, slot);
+  prefill_tile_serial<D, T, TT, G, TP>(p, s, b, h, rt, 0, kAllSteps, 0);
 }
 
 // One part of the balanced grid per block (blocks past the last exit; an
@@ -1062,26 +1052,29 @@ __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) vo
   const int n = p.balanced_blocks;
   const int x = n % kXcds == 0 ? (int)(blockIdx.x % kXcds) * (n / kXcds) + (int)(blockIdx.x / kXcds) : (int)blockIdx.x;
   for (int i = x;; i += n) {
-    // (Looked up again for each of an unsplit call's tiles: kept over the tile,
-    // the lookup's values would spill.)
+    // (Scanned again for each of an unsplit call's tiles: kept over the tile,
+    // its lanes' values would spill.)
+    const CallParts<TT, G> parts(p);
+    const bool more = !parts.split();
     PartPos w;
-    bool split;
-    if (!find_part<Find::kPart, TT, G>(p, i, w, split)) return;
-    const PartSteps steps = part_steps<TT, G>(p, w.s, w.rt, w.parts, w.part);
-    if (steps.begin < steps.end)
-      prefill_tile_serial<D, T, TT, G, TP>(p, w.s, w.b, w.h, w.rt, steps.begin, steps.end,
+    if (!parts.template find<Find::kPart>(p, i, w)) return;
+    const int own = (block_key_tiles<TT>(w.s, p.group_size, w.rt) + G - 1) / G; // steps the tile's rows see
+    const int k = min(w.parts, own);
+    if (w.part < k)
+      prefill_tile_serial<D, T, TT, G, TP>(p, w.s, w.b, w.h, w.rt, (unsigned)(w.part * own) / (unsigned)k,
+                                           (unsigned)((w.part + 1) * own) / (unsigned)k,
                                            w.slot0 + w.part * seq_row_tiles(p, w.s));
-    if (split) return;
+    if (!more) return;
     __syncthreads(); // group 0's hand-off reads end before the next tile refills the stages
   }
 }
 
-// Merges the parts of a split grid's tiles:
+// Merges the parts of the balanced grid's tiles:
 //   out = sum_j 2^(m_j - M) o_j / sum_j 2^(m_j - M) l_j,  M = max_j m_j.
 // A wavefront takes the 32 rows of one row wavefront, in the partials' register
 // layout (lane l: row l % 32), and of their dims one float4 per lane (F16: 8
 // consecutive dims of a row) or D / 32 (F32: as many consecutive dims per lane
-// and element).  16 parts (F32: 8), weights and rows, are in flight at once: the
+// and element).  8 parts (F32: 4), weights and rows, are in flight at once: the
 // kernel is bound by its dependent round trips (lengths, then the parts).
 template <int D, bool kF32>
 constexpr int merge_waves_per_tile() {
@@ -1092,64 +1085,43 @@ __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(Prefill
   constexpr int TT = prefill_tile_tokens<D, T>();
   constexpr bool kF32 = sizeof(T) == 4;
   constexpr int kVecs = kF32 ? D / 32 : 1; // float4 per lane
-  constexpr int kBatch = kF32 ? 8 : 16;    // parts in flight
+  constexpr int kBatch = kF32 ? 4 : 8;     // parts in flight
   constexpr int kPerTile = merge_waves_per_tile<D, kF32>();
   static_assert(kPerTile % kMergeWaves == 0, "whole blocks per tile");
-  const int tile = blockIdx.x / (kPerTile / kMergeWaves);
+  const CallParts<TT, G> call(p);
+  PartPos t;
+  if (!call.split() || !call.template find<Find::kTile>(p, blockIdx.x / (kPerTile / kMergeWaves), t)) return;
+  const int own = (block_key_tiles<TT>(t.s, p.group_size, t.rt) + G - 1) / G; // steps its rows see
+  const int parts = min(t.parts, own);
+  if (parts <= 1) return;
+  const int rts = seq_row_tiles(p, t.s);
   const int l = threadIdx.x & 63;
   const int hh = l >> 5;
   const int unit = blockIdx.x % (kPerTile / kMergeWaves) * kMergeWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rw = unit % kRowWaves, k = unit / kRowWaves; // k: n * 4 + e / 4 (F16) or e / 4 (F32)
-  // The tile's slots: part j's is slot0 + j * stride, `slots` of them exist.
-  PartPos t;
-  int stride = 1, slots = p.kv_splits;
-  if (p.balanced_blocks > 0) {
-    bool split;
-    if (!find_part<Find::kTile, TT, G>(p, tile, t, split) || !split) return;
-    stride = seq_row_tiles(p, t.s);
-    slots = t.parts;
-  } else {
-    t.slot0 = tile * p.kv_splits;
-    t.rt = tile % p.row_tiles;
-    t.h = tile / p.row_tiles % p.num_kv_heads;
-    t.b = p.seq_lo + tile / (p.row_tiles * p.num_kv_heads);
-  }
+  const int rho = t.rt * kBlockRows + rw * kRowsPerWave + (l & 31);
+  const bool valid = rho < p.group_size * t.s.q_len;
   const float2v* ml = reinterpret_cast<const float2v*>(p.partial_ml) + (int64_t)t.slot0 * kBlockRows + rw * kRowsPerWave + (l & 31);
   const float4v* src = reinterpret_cast<const float4v*>(p.partial_o) +
                        ((int64_t)t.slot0 * kRowWaves + rw) * (D / 8 * 64) + k * 64 + l;
-  // One batch of parts; slots past the last repeat it, and those that hold
-  // nothing of this call get weight 0 below.  The first batch is requested
-  // before the tile's bounds are known.
-  float2v mlj[kBatch] = {};
-  float4v o[kBatch][kVecs] = {};
-  auto load_batch = [&](int j0) {
-#pragma unroll
-    for (int u4 = 0; u4 < kBatch; u4 += 4) {
-      if (u4 > 0 && j0 + u4 >= slots) break; // (wave-uniform; the weights below skip what was not loaded)
-#pragma unroll
-      for (int u = u4; u < u4 + 4; u++) {
-        const int64_t j = (int64_t)min(j0 + u, slots - 1) * stride;
-        mlj[u] = ml[j * kBlockRows];
-#pragma unroll
-        for (int v = 0; v < kVecs; v++) o[u][v] = src[j * kRowWaves * (D / 8 * 64) + 4 * v * 64];
-      }
-    }
-  };
-  load_batch(0);
-  if (p.balanced_blocks == 0) t.s = load_rows(p, t.b);
-  const int parts = part_steps<TT, G>(p, t.s, t.rt, slots, 0).parts;
-  if (parts <= 1) return;
-  const int rho = t.rt * kBlockRows + rw * kRowsPerWave + (l & 31);
-  const bool valid = rho < p.group_size * t.s.q_len;
   float m = -INFINITY, den = 0.f;
   float4v acc[kVecs];
 #pragma unroll
   for (int v = 0; v < kVecs; v++) acc[v] = float4v{0.f, 0.f, 0.f, 0.f};
   for (int j0 = 0; j0 < parts; j0 += kBatch) {
-    if (j0 > 0) load_batch(j0);
+    // (Past the last part: its rows again, at weight 0.)
+    float2v mlj[kBatch];
+    float4v o[kBatch][kVecs];
+#pragma unroll
+    for (int u = 0; u < kBatch; u++) {
+      const int64_t j = min(j0 + u, parts - 1) * rts;
+      mlj[u] = ml[j * kBlockRows];
+#pragma unroll
+      for (int v = 0; v < kVecs; v++) o[u][v] = src[j * kRowWaves * (D / 8 * 64) + 4 * v * 64];
+    }
     float m_new = m;
 #pragma unroll
-    for (int u = 0; u < kBatch; u++) m_new = fmaxf(m_new, j0 + u < parts ? mlj[u][0] : -INFINITY);
+    for (int u = 0; u < kBatch; u++) m_new = fmaxf(m_new, mlj[u][0]);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const float alpha = __builtin_amdgcn_exp2f(m - m_use); // 0 in the first batch
     den *= alpha;
@@ -1158,7 +1130,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(Prefill
 #pragma unroll
     for (int u = 0; u < kBatch; u++) {
       const float w = j0 + u < parts ? __builtin_amdgcn_exp2f(mlj[u][0] - m_use) : 0.f; // m = -inf (no visible key): 0
-      den += w == 0.f ? 0.f : w * mlj[u][1];
+      den += w * mlj[u][1];
 #pragma unroll
       for (int v = 0; v < kVecs; v++)
 #pragma unroll
@@ -1191,30 +1163,24 @@ __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(Prefill
 
 template <int D, typename T, int G, bool TP>
 hipError_t launch_shape(const PrefillParams& params, hipStream_t stream) {
-  // (One-group blocks up to D=128 are for grids of many blocks per CU: unsplit.)
-  constexpr bool kSplits = G == 2 || D > 128;
-  if (!kSplits && (params.balanced_blocks > 0 || params.kv_splits > 1)) return hipErrorInvalidValue;
-  int64_t tiles = params.balanced_tiles;
   if (params.balanced_blocks > 0) {
-    if constexpr (kSplits)
+    // (One-group blocks up to D=128 are for grids of many blocks per CU.)
+    if constexpr (G == 1 && D <= 128) {
+      return hipErrorInvalidValue;
+    } else {
       hipLaunchKernelGGL((paged_prefill_balanced_kernel<D, T, G, TP>), dim3((unsigned)params.balanced_blocks),
                          dim3(kRowWaves * G * 64), 0, stream, params);
+      const hipError_t err = hipGetLastError();
+      if (err != hipSuccess) return err;
+      hipLaunchKernelGGL((prefill_merge_kernel<D, T, G>),
+                         dim3((unsigned)(params.balanced_tiles * (merge_waves_per_tile<D, sizeof(T) == 4>() / kMergeWaves))),
+                         dim3(64 * kMergeWaves), 0, stream, params);
+    }
   } else {
     const int64_t blocks = prefill_main_blocks(params) + params.catch_count;
-    if (kSplits && params.kv_splits > 1)
-      hipLaunchKernelGGL((paged_prefill_kernel<D, T, G, TP, kSplits>), dim3((unsigned)blocks), dim3(kRowWaves * G * 64),
-                         0, stream, params);
-    else
-      hipLaunchKernelGGL((paged_prefill_kernel<D, T, G, TP, false>), dim3((unsigned)blocks), dim3(kRowWaves * G * 64),
-                         0, stream, params);
-    tiles = (int64_t)(params.seq_count ? params.seq_count : params.num_seqs) * params.num_kv_heads * params.row_tiles;
+    hipLaunchKernelGGL((paged_prefill_kernel<D, T, G, TP>), dim3((unsigned)blocks), dim3(kRowWaves * G * 64), 0,
+                       stream, params);
   }
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess || (params.balanced_blocks == 0 && params.kv_splits == 1)) return err;
-  if constexpr (kSplits)
-    hipLaunchKernelGGL((prefill_merge_kernel<D, T, G>),
-                       dim3((unsigned)(tiles * (merge_waves_per_tile<D, sizeof(T) == 4>() / kMergeWaves))),
-                       dim3(64 * kMergeWaves), 0, stream, params);
   return hipGetLastError();
 }
 
