@@ -311,22 +311,21 @@ bool longest_first_pays(const mvr_paged_attention_args* a, const LiveSeqs& live)
   constexpr int kBlockTokens = 128; // a block's cost beside its keys, in tokens
   const int cus = device_cus();
   const int per_round = cus / a->num_kv_heads; // sequences whose tiles the CUs hold at once
-  if (per_round < 1 || a->num_seqs <= per_round) return false;
-  std::vector<int> cost;
-  cost.reserve(a->num_seqs);
-  int64_t sum = 0;
+  constexpr int kMaxRanked = 4096; // on the stack: planning allocates nothing
+  if (per_round < 1 || a->num_seqs <= per_round || a->num_seqs > kMaxRanked) return false;
+  int cost[kMaxRanked];
+  int64_t n = 0, sum = 0;
   for (int s = 0; s < a->num_seqs; s++) {
     const int q = live.cu_q_lens[s + 1] - live.cu_q_lens[s];
     if (q < live.q_min || q > live.q_max) continue;
-    cost.push_back(std::max(live.seq_lens[s] - live.key_begin, 0) + kBlockTokens);
-    sum += cost.back();
+    cost[n] = std::max(live.seq_lens[s] - live.key_begin, 0) + kBlockTokens;
+    sum += cost[n++];
   }
-  const int64_t n = (int64_t)cost.size();
   if (n <= per_round || sum < n * (768 + kBlockTokens)) return false;
-  std::nth_element(cost.begin(), cost.begin() + per_round, cost.end(), std::greater<int>());
+  std::nth_element(cost, cost + per_round, cost + n, std::greater<int>());
   const int next = cost[per_round]; // the (per_round + 1)-th longest
-  const int last = *std::min_element(cost.begin(), cost.begin() + per_round);
-  const int longest = *std::max_element(cost.begin(), cost.begin() + per_round);
+  const int last = *std::min_element(cost, cost + per_round);
+  const int longest = *std::max_element(cost, cost + per_round);
   const double load = (double)sum * a->num_kv_heads / cus;
   return load >= 0.7 * std::max({(double)longest, load, (double)last + next});
 }
