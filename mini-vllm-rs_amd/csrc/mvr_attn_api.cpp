@@ -187,6 +187,9 @@ struct LiveSeqs {
   int q_min = 1, q_max = INT32_MAX, key_begin = 0;
   // Largest workspace the balanced prefill grid's partials may take.
   size_t prefill_budget = (size_t)48 << 20;
+  // The split-context kernel's partials do not fit the workspace given: take
+  // the plan that keeps none, where one exists.
+  bool no_partials = false;
 };
 
 // Keys of one step of a prefill block: one key tile of 64 tokens (F32: 32)
@@ -307,7 +310,6 @@ void plan_balanced(const mvr_paged_attention_args* a, const LiveSeqs& live, int6
 // 382 us on the first two.
 bool longest_first_pays(const mvr_paged_attention_args* a, const LiveSeqs& live) {
   if (!live.seq_lens || !live.cu_q_lens) return false;
-  if (a->head_dim * (a->dtype == MVR_DTYPE_F16 ? 2 : 4) < 256) return false;
   constexpr int kBlockTokens = 128; // a block's cost beside its keys, in tokens
   const int cus = device_cus();
   const int per_round = cus / a->num_kv_heads; // sequences whose tiles the CUs hold at once
@@ -481,9 +483,13 @@ mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_
       if (plan.max_parts <= w && 4 * plan.max_parts >= 3 * w) plan.block_waves = w;
   }
   static const bool dense_enabled = env_bool("MVR_ATTN_DENSE_RAGGED", true);
-  const bool longest_first = block_merge_enabled && dense_enabled && cpp_override_none && ragged &&
+  // (Rows of at least 256 bytes: longest_first_pays.)  Correct for any tables
+  // and without partials, it is also what a call falls back to whose workspace
+  // was sized for tables that took it.
+  const bool longest_first = block_merge_enabled && dense_enabled && cpp_override_none && a->sum_seq_lens > 0 &&
                              plan.row_blocks == 1 && plan.row_tiles == 1 && all_plans && !plan.token_pages &&
-                             longest_first_pays(a, live);
+                             a->head_dim * (a->dtype == MVR_DTYPE_F16 ? 2 : 4) >= 256 &&
+                             (live.no_partials || (ragged && longest_first_pays(a, live)));
   if (longest_first) {
     plan.block_waves = 8; // each tile's chunks split evenly over the block
     plan.max_parts = 8;
@@ -792,12 +798,14 @@ struct CallPlan {
   size_t total = 0;
 };
 
-// budget: the largest workspace of the prefill launch's partials.
-CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget) {
+// budget: the largest workspace of the prefill launch's partials; no_partials:
+// the split-context launch keeps none where it can.
+CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget, bool no_partials = false) {
   CallPlan c;
   c.part[0] = *a;
   LiveSeqs all;
   all.prefill_budget = budget;
+  all.no_partials = no_partials;
   use_tables(a, 1, INT32_MAX, all);
   c.plan[0] = make_plan(a, true, all);
   c.total = c.plan[0].partial_bytes;
@@ -865,6 +873,7 @@ CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget) {
   p0.max_q_len = qmax;
   LiveSeqs live0;
   live0.count = count[0];
+  live0.no_partials = no_partials;
   if (hinted) {
     if (sl) live0.max_seq_len = lmax[0];
     use_tables(a, 1, qmax, live0);
@@ -910,15 +919,20 @@ CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget) {
   return c;
 }
 
-// The call's plan in `limit` bytes of workspace, `used` of them taken: where
-// the balanced prefill grid's partials do not fit, it gets fewer blocks, down
-// to none (the unsplit grid, which needs no workspace).
+// The call's plan in `limit` bytes of workspace, `used` of them taken.  What a
+// call needs varies with the host tables, and a workspace may have been sized
+// for others: where the balanced prefill grid's partials do not fit, it gets
+// fewer blocks, down to none (the unsplit grid, which needs no workspace); then
+// the split-context launch drops its own where it can (longest first).
 CallPlan make_call_plan(const mvr_paged_attention_args* a, size_t limit = SIZE_MAX, size_t used = 0) {
   CallPlan c = plan_call_within(a, LiveSeqs{}.prefill_budget);
-  const mvr::PagedAttentionPlan& last = c.plan[c.n - 1];
-  if (last.prefill && used + c.total > limit) {
+  for (bool no_partials : {false, true}) {
+    if (used + c.total <= limit) break;
+    if (no_partials) c = plan_call_within(a, LiveSeqs{}.prefill_budget, true);
+    const mvr::PagedAttentionPlan& last = c.plan[c.n - 1];
+    if (!last.prefill || used + c.total <= limit) continue;
     const size_t other = used + c.total - last.partial_bytes + 512; // alignment of the two partial arrays
-    c = plan_call_within(a, limit > other ? limit - other : 0);
+    c = plan_call_within(a, limit > other ? limit - other : 0, no_partials);
   }
   return c;
 }
@@ -1075,10 +1089,17 @@ CascadePlan make_cascade_plan(const mvr_paged_attention_args* a, const mvr_casca
   if (c.suf.sum_seq_lens >= suf_len * a->num_seqs) c.suf.sum_seq_lens = 0;
   // The suffix pass starts every sequence at its prefix: split-context kernel.
   c.suf_plan = make_plan(&c.suf, /*allow_prefill=*/false, suf_live);
+  // The tables may have chosen a plan without partials; others may not: the
+  // workspace holds what the same call needs without them.
+  size_t suf_bytes = c.suf_plan.partial_bytes;
+  if (suf_live.seq_lens) {
+    suf_live.seq_lens = suf_live.cu_q_lens = nullptr;
+    suf_bytes = std::max(suf_bytes, make_plan(&c.suf, /*allow_prefill=*/false, suf_live).partial_bytes);
+  }
   const size_t so = (size_t)a->num_q_heads * c.state_tokens * a->head_dim * sizeof(float);
   const size_t sl = (size_t)a->num_q_heads * c.state_tokens * sizeof(float);
   c.off_suf = align_up(c.pre_plan.partial_bytes, 256);
-  c.off_a_o = c.off_suf + align_up(c.suf_plan.partial_bytes, 256);
+  c.off_a_o = c.off_suf + align_up(suf_bytes, 256);
   c.off_a_lse = c.off_a_o + align_up(so, 256);
   c.total = c.off_a_lse + align_up(sl, 256);
   return c;
