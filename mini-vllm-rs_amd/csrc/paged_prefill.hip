@@ -886,88 +886,86 @@ struct PartPos {
   int b, h, rt, part, parts, slot0; // slot0: the slot of the tile's part 0; part j's is slot0 + j * row tiles
 };
 
-// 64 sequences from b0 on, one per lane: the parts of each, their inclusive
-// sum and total (nothing past the last sequence or for another launch's).
+// Row tiles of a sequence over all KV heads, and parts per tile.
 template <int TT, int G>
-struct SeqParts {
-  SeqRows s;
-  int per_tile, tiles, incl, total, tiles_incl;
-  __device__ __forceinline__ SeqParts(const PrefillParams& p, int b0, bool split) : per_tile(0), tiles(0) {
-    const int b = b0 + (int)(threadIdx.x & 63);
-    s = load_lane_rows(p, min(b, p.num_seqs - 1));
-    if (b < p.num_seqs && s.q_len > 0 && s.key_end > 0) {
-      tiles = p.num_kv_heads * seq_row_tiles(p, s);
-      const int steps = (s.key_end + G * TT - 1) / (G * TT);
-      per_tile = split ? min((int)((unsigned)(steps + p.part_steps - 1) / (unsigned)p.part_steps), kMaxParts) : 1;
-    }
-    incl = wave_inclusive_sum(per_tile * tiles);
-    total = __builtin_amdgcn_readlane(incl, 63);
-    tiles_incl = wave_inclusive_sum(tiles);
-  }
-};
+__device__ __forceinline__ void seq_parts(const PrefillParams& p, const SeqRows& s, bool split, int& tiles,
+                                          int& per_tile) {
+  tiles = s.q_len > 0 && s.key_end > 0 ? p.num_kv_heads * seq_row_tiles(p, s) : 0;
+  const unsigned steps = (unsigned)(max(s.key_end, 0) + G * TT - 1) / (G * TT);
+  per_tile = split ? min((int)((steps + p.part_steps - 1) / (unsigned)p.part_steps), kMaxParts) : 1;
+}
 
-// The call's parts; the first 64 sequences' stay in registers.
-template <int TT, int G>
-class CallParts {
-  bool split_;
-  SeqParts<TT, G> head_;
-  int total_, tiles_;
-  __device__ __forceinline__ void sum(const PrefillParams& p) {
-    total_ = head_.total;
-    tiles_ = lane(head_.tiles_incl, 63);
-    for (int b0 = 64; b0 < p.num_seqs; b0 += 64) {
-      const SeqParts<TT, G> c(p, b0, split_);
-      total_ += c.total;
-      tiles_ += lane(c.tiles_incl, 63);
-    }
+// Part (or tile) `rel` of w.s, whose parts start at slot `slot`.
+template <Find kFind>
+__device__ __forceinline__ void place(const PrefillParams& p, int rel, int slot, PartPos& w) {
+  const int rts = seq_row_tiles(p, w.s);
+  if (kFind == Find::kPart) {
+    w.h = (unsigned)rel / (unsigned)(w.parts * rts);
+    const int in_head = rel - w.h * w.parts * rts;
+    w.part = (unsigned)in_head / (unsigned)rts;
+    w.rt = in_head - w.part * rts;
+  } else {
+    w.h = (unsigned)rel / (unsigned)rts;
+    w.part = 0;
+    w.rt = rel - w.h * rts;
   }
-  __device__ __forceinline__ static int lane(int v, int src) { return __builtin_amdgcn_readlane(v, src); }
+  w.slot0 = slot + w.h * w.parts * rts + w.rt;
+}
 
- public:
-  __device__ __forceinline__ explicit CallParts(const PrefillParams& p) : split_(true), head_(p, 0, true) {
-    sum(p);
-    if (total_ > p.balanced_blocks || tiles_ > p.balanced_tiles) {
-      split_ = false;
-      head_ = SeqParts<TT, G>(p, 0, false);
-      sum(p);
-    }
-  }
-  __device__ __forceinline__ bool split() const { return split_; }
-  // Part i, or (kTile) part 0 of tile i; false past the last one.
-  template <Find kFind>
-  __device__ __forceinline__ bool find(const PrefillParams& p, int i, PartPos& w) const {
-    int slot = 0;
+// Part i of the call, or (kTile) part 0 of its tile i; false past the last
+// one.  `split`: whether the call is split at all.  The sequences are scanned
+// 64 at a time, one per lane.  (Up to 8 sequences walked with scalar loads
+// instead: 189 against 182 us on three ragged F32 chunks.)
+template <Find kFind, int TT, int G>
+__device__ __forceinline__ bool find_part(const PrefillParams& p, int i, PartPos& w, bool& split) {
+  split = true;
+  auto lane = [](int v, int src) { return __builtin_amdgcn_readlane(v, src); };
+  for (;;) {
+    int left = i, rel = -1, slot0 = 0, slots = 0, all_tiles = 0;
     for (int b0 = 0; b0 < p.num_seqs; b0 += 64) {
-      const SeqParts<TT, G> c = b0 == 0 ? head_ : SeqParts<TT, G>(p, b0, split_);
-      const int incl = kFind == Find::kPart ? c.incl : c.tiles_incl;
-      const int n = kFind == Find::kPart ? c.per_tile * c.tiles : c.tiles;
+      const int b = b0 + (int)(threadIdx.x & 63);
+      const SeqRows s = load_lane_rows(p, min(b, p.num_seqs - 1));
+      int tiles, per_tile;
+      seq_parts<TT, G>(p, s, split, tiles, per_tile);
+      if (b >= p.num_seqs) tiles = 0;
+      const int parts_incl = wave_inclusive_sum(per_tile * tiles), tiles_incl = wave_inclusive_sum(tiles);
+      const int incl = kFind == Find::kPart ? parts_incl : tiles_incl;
       const int total = lane(incl, 63);
-      if (i < total) {
-        const int src = __builtin_ctzll(__ballot(i < incl));
-        const int rel = i - lane(incl - n, src);
-        w.s = SeqRows{lane(c.s.seq_len, src), lane(c.s.q_start, src), lane(c.s.q_len, src), lane(c.s.key_end, src)};
+      if (rel < 0 && left < total) {
+        const int src = __builtin_ctzll(__ballot(left < incl));
+        w.s = SeqRows{lane(s.seq_len, src), lane(s.q_start, src), lane(s.q_len, src), lane(s.key_end, src)};
         w.b = b0 + src;
-        w.parts = lane(c.per_tile, src);
-        const int rts = seq_row_tiles(p, w.s);
-        if (kFind == Find::kPart) {
-          w.h = (unsigned)rel / (unsigned)(w.parts * rts);
-          const int in_head = rel - w.h * w.parts * rts;
-          w.part = (unsigned)in_head / (unsigned)rts;
-          w.rt = in_head - w.part * rts;
-        } else {
-          w.h = (unsigned)rel / (unsigned)rts;
-          w.part = 0;
-          w.rt = rel - w.h * rts;
-        }
-        w.slot0 = slot + lane(c.incl - c.per_tile * c.tiles, src) + w.h * w.parts * rts + w.rt;
-        return true;
+        w.parts = lane(per_tile, src);
+        rel = left - lane(incl - (kFind == Find::kPart ? per_tile * tiles : tiles), src);
+        slot0 = slots + lane(parts_incl - per_tile * tiles, src);
       }
-      i -= total;
-      slot += c.total;
+      left -= total;
+      slots += lane(parts_incl, 63);
+      all_tiles += lane(tiles_incl, 63);
     }
-    return false;
+    if (split && (slots > p.balanced_blocks || all_tiles > p.balanced_tiles)) {
+      split = false;
+      continue;
+    }
+    if (rel < 0) return false;
+    place<kFind>(p, rel, slot0, w);
+    return true;
   }
+}
+
+// Steps of part `part` of a tile in `parts` parts: an even share of the steps
+// that its rows see (fewer parts than that many hold any).
+struct PartSteps {
+  int begin, end, parts; // parts that hold steps
 };
+template <int TT, int G>
+__device__ __forceinline__ PartSteps part_steps(const PrefillParams& p, const SeqRows& s, int rt, int parts, int part) {
+  const int own = (block_key_tiles<TT>(s, p.group_size, rt) + G - 1) / G;
+  const int k = min(parts, own);
+  if (part >= k) return {0, 0, k};
+  const int each = (unsigned)own / (unsigned)k, rest = own - each * k; // the first `rest` parts take one more
+  return {part * each + min(part, rest), (part + 1) * each + min(part + 1, rest), k};
+}
 
 // Main grid: block x covers (sequence, kv head, row tile) of the main range,
 // unsplit.  XCD-aware decode: block x runs on XCD x % 8 and all blocks of one
@@ -1052,19 +1050,16 @@ __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) vo
   const int n = p.balanced_blocks;
   const int x = n % kXcds == 0 ? (int)(blockIdx.x % kXcds) * (n / kXcds) + (int)(blockIdx.x / kXcds) : (int)blockIdx.x;
   for (int i = x;; i += n) {
-    // (Scanned again for each of an unsplit call's tiles: kept over the tile,
-    // its lanes' values would spill.)
-    const CallParts<TT, G> parts(p);
-    const bool more = !parts.split();
+    // (Looked up again for each of an unsplit call's tiles: kept over the tile,
+    // the lookup's values would spill.)
     PartPos w;
-    if (!parts.template find<Find::kPart>(p, i, w)) return;
-    const int own = (block_key_tiles<TT>(w.s, p.group_size, w.rt) + G - 1) / G; // steps the tile's rows see
-    const int k = min(w.parts, own);
-    if (w.part < k)
-      prefill_tile_serial<D, T, TT, G, TP>(p, w.s, w.b, w.h, w.rt, (unsigned)(w.part * own) / (unsigned)k,
-                                           (unsigned)((w.part + 1) * own) / (unsigned)k,
+    bool split;
+    if (!find_part<Find::kPart, TT, G>(p, i, w, split)) return;
+    const PartSteps steps = part_steps<TT, G>(p, w.s, w.rt, w.parts, w.part);
+    if (steps.begin < steps.end)
+      prefill_tile_serial<D, T, TT, G, TP>(p, w.s, w.b, w.h, w.rt, steps.begin, steps.end,
                                            w.slot0 + w.part * seq_row_tiles(p, w.s));
-    if (!more) return;
+    if (split) return;
     __syncthreads(); // group 0's hand-off reads end before the next tile refills the stages
   }
 }
@@ -1088,11 +1083,10 @@ __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(Prefill
   constexpr int kBatch = kF32 ? 4 : 8;     // parts in flight
   constexpr int kPerTile = merge_waves_per_tile<D, kF32>();
   static_assert(kPerTile % kMergeWaves == 0, "whole blocks per tile");
-  const CallParts<TT, G> call(p);
   PartPos t;
-  if (!call.split() || !call.template find<Find::kTile>(p, blockIdx.x / (kPerTile / kMergeWaves), t)) return;
-  const int own = (block_key_tiles<TT>(t.s, p.group_size, t.rt) + G - 1) / G; // steps its rows see
-  const int parts = min(t.parts, own);
+  bool split;
+  if (!find_part<Find::kTile, TT, G>(p, blockIdx.x / (kPerTile / kMergeWaves), t, split) || !split) return;
+  const int parts = part_steps<TT, G>(p, t.s, t.rt, t.parts, 0).parts;
   if (parts <= 1) return;
   const int rts = seq_row_tiles(p, t.s);
   const int l = threadIdx.x & 63;
