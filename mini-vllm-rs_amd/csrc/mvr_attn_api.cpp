@@ -185,7 +185,8 @@ struct LiveSeqs {
   const int32_t* cu_q_lens = nullptr;
   const int32_t* seq_lens = nullptr;
   int q_min = 1, q_max = INT32_MAX, key_begin = 0;
-  // Largest workspace the balanced prefill grid's partials may take.
+  int64_t span = 0; // prefill kernel: sequences of the main grid (0: num_seqs)
+  // Largest workspace a split prefill grid's partials may take.
   size_t prefill_budget = (size_t)48 << 20;
   // The split-context kernel's partials do not fit the workspace given: take
   // the plan that keeps none, where one exists.
@@ -198,21 +199,29 @@ int prefill_step_keys(const mvr_paged_attention_args* a) {
   return (a->dtype == MVR_DTYPE_F16 ? 64 : 32) * (a->head_dim > 128 ? 1 : 2);
 }
 
-// Balanced prefill grid (each row tile's keys in parts of at most part_steps
-// steps, a block per part, and a merge launch) where the unsplit one, a block
-// per row tile, leaves CUs idle or waits for its longest sequence.
-// For one to four rounds of blocks over the CUs, and for fewer parts that leave
-// CUs idle: the shortest parts whose blocks fit, and their estimated time.
-// Measured at D=128 (one box, HIP events): a step of the two-group block takes
-// 1.5 us in F16 and 6.9 us in F32 alone and 0.5 / 0.9 us more with every CU
-// busy; a block costs 8 us beside its steps; a split call 5 us for the merge
-// and 11 us per CU-full of parts for their partial rows (64 KiB each, written
-// and read) and their cold start.  F16, 256 tokens on 2,048, 64 tiles: 37.0 us
-// unsplit, 36.1 / 33.7 / 36.0 in 2 / 3 / 4 parts; 64 on 8,128, 16 tiles: 102.7,
-// and 51.5 / 41.4 / 33.7 / 29.7 in 3 / 4 / 6 / 8; F32, 3 x 217 tokens on
-// 897..2,320: 309 unsplit, 168 in parts of at most 20 steps.
-void plan_balanced(const mvr_paged_attention_args* a, const LiveSeqs& live, int64_t n_live, int len_live,
-                   mvr::PagedAttentionPlan& plan) {
+// Split prefill grids, where the unsplit one, a block per row tile, leaves CUs
+// idle or waits for its longest sequence: each tile's keys in parts, a block
+// per part, and a merge launch.  Either every tile of the main grid in kv_splits
+// parts, whose blocks and merge find theirs from the block index, or, for
+// sequences of unequal lengths, the balanced grid's parts of at most part_steps
+// steps, found by a scan of the length tables.  Both are priced, the balanced
+// grid for one to four rounds of blocks over the CUs and for fewer parts that
+// leave CUs idle (the shortest parts whose blocks fit).
+// Measured (one box, HIP events, 47 calls of one length, each in 1..32 parts;
+// F16 and F32, D=64..256, 17..1,024 new tokens on 0..16,000): a step of the
+// two-group block takes 1.45 us in F16 at D=128 (0.57 of that at D=64: its
+// softmax does not shrink), 0.85 us more with every CU busy, and 7.7 / 0.65 us
+// in F32; a block costs 7.2 us beside its steps; the merge launch 4 us, 1.5 us
+// more from 64 tiles on and 2.5 us per 8 parts after the first 8; the balanced
+// grid's scans 3 us more.  The parts chosen so took 0.9% longer than the best on
+// average, at most 5% (one case of 13% at D=256).  F16, 256 tokens on 2,048, 64
+// tiles: 35.4 us unsplit, 29.3 / 26.4 / 26.4 / 35.6 in 2 / 3 / 4 / 5 parts; 64
+// on 8,128, 16 tiles: 102.6, and 36.4 / 25.9 / 24.4 / 33.1 in 4 / 8 / 16 / 20;
+// D=64, 2 x 153 on 600, 80 tiles: 13.3, 16.8 in 2; F32, 256 on 2,048, 56 tiles:
+// 278, 87.1 / 130 in 4 / 5; 3 x 217 on 897..2,320: 309, 168 in parts of at most
+// 20 steps.
+void plan_prefill_splits(const mvr_paged_attention_args* a, const LiveSeqs& live, int64_t n_live, int len_live,
+                         mvr::PagedAttentionPlan& plan) {
   const int64_t cus = device_cus();
   const int group = a->num_q_heads / a->num_kv_heads;
   const int step_keys = prefill_step_keys(a);
@@ -230,7 +239,9 @@ void plan_balanced(const mvr_paged_attention_args* a, const LiveSeqs& live, int6
     }
   };
   int64_t tiles = 0, steps = 0, longest = 0;
+  bool equal = true; // sequences of one number of steps
   each([&](int64_t t, int64_t n) {
+    equal = equal && (tiles == 0 || n == longest);
     tiles += t;
     steps += t * n;
     longest = std::max(longest, n);
@@ -250,45 +261,83 @@ void plan_balanced(const mvr_paged_attention_args* a, const LiveSeqs& live, int6
   const bool f16 = a->dtype == MVR_DTYPE_F16;
   const size_t slot_bytes = (size_t)mvr::kPrefillBlockRows * (a->head_dim + 2) * sizeof(float);
   const int64_t slots = (int64_t)(live.prefill_budget / slot_bytes);
-  static const int split_override = env_int("MVR_ATTN_PREFILL_SPLITS", 0);
-  auto cost_us = [&](int64_t blocks, int64_t part) {
+  const double dims = a->head_dim / 128.0;
+  // `blocks` of at most `part` steps; `share`: the busiest XCD's blocks over an
+  // even share of them.
+  auto cost_us = [&](int64_t blocks, double part, double share) {
     const double fill = std::min(1.0, (double)blocks / cus);
-    const double step = ((f16 ? 1.5 : 6.9) + (f16 ? 0.5 : 0.9) * fill) * a->head_dim / 128;
-    const double load = blocks <= cus ? (double)part : std::max((double)part, (double)steps / cus + part / 2);
-    return load * step + 8.0 * ((blocks + cus - 1) / cus);
+    const double step = f16 ? (1.45 + 0.85 * fill) * (0.13 + 0.87 * dims) : (7.7 + 0.65 * fill) * dims;
+    const double busy = blocks * share;
+    const double load = busy <= cus ? part : std::max(part, share * steps / cus + part / 2);
+    return load * step + 7.2 * ceil(busy / cus);
   };
-  double best = split_override > 1 ? INFINITY : 0.97 * cost_us(tiles, longest);
-  int64_t best_part = 0;
-  for (int64_t quarters : {1, 2, 3, 4, 8, 12, 16}) { // of a block per CU
-    const int64_t most = std::min(split_override > 1 ? tiles * split_override : quarters * cus / 4, slots);
-    if (split_override == 1 || most < tiles) continue;
-    int64_t lo = std::min<int64_t>(2, longest), hi = longest; // blocks_at(hi) = tiles <= most
-    while (lo < hi) {
-      const int64_t mid = (lo + hi) / 2;
-      if (blocks_at(mid) <= most)
-        hi = mid;
-      else
-        lo = mid + 1;
-    }
-    if (lo >= longest) continue;
-    int64_t part = 0;
-    const int64_t blocks = blocks_at(lo, &part);
-    const double cost = cost_us(blocks, part) + 5 + 11.0 * blocks / cus * a->head_dim / 128;
+  auto merge_us = [&](int64_t parts) {
+    return 4.0 + 1.5 * std::min(1.0, tiles / 64.0) + 2.5 * ((parts - 1) / 8);
+  };
+  // The main grid deals whole (sequence, KV head) pairs to the 8 XCDs: 12 pairs
+  // put two on four of them (3 x 50 F16 tokens on 3,000, 36 tiles: 24.1 us in 5
+  // parts, 35.0 in 6, whose 36 blocks per XCD need a second round).
+  const int64_t span = live.span > 0 && live.span < a->num_seqs ? live.span : a->num_seqs;
+  const int64_t span_tiles = span * a->num_kv_heads * plan.row_tiles;
+  const int64_t pairs = span * a->num_kv_heads;
+  const double share = tiles == span_tiles && pairs >= 8 ? 8.0 * ((pairs + 7) / 8) / pairs : 1.0;
+  static const int split_override = env_int("MVR_ATTN_PREFILL_SPLITS", 0);
+  if (split_override == 1) return;
+  double best = split_override > 1 ? INFINITY : cost_us(tiles, longest, share);
+  // As many parts for every tile: up to a block per CU, or any number of rounds
+  // for sequences of one length.
+  const int64_t most_parts = std::min<int64_t>(
+      {longest, (int64_t)mvr::kPrefillMaxParts, slots / span_tiles, (equal ? 4 : 1) * cus / tiles,
+       split_override > 1 ? split_override : INT32_MAX});
+  const int64_t groups = a->head_dim > 128 ? 1 : 2; // key tiles per step: its parts end at any tile
+  int64_t splits = 1;
+  for (int64_t k = split_override > 1 ? most_parts : 2; k <= most_parts && k > 1; k++) {
+    const double cost = cost_us(tiles * k, (double)((longest * groups + k - 1) / k) / groups, share) + merge_us(k);
     if (cost < best) {
       best = cost;
-      best_part = lo;
+      splits = k;
     }
-    if (split_override > 1) break;
   }
-  // (Part counts are 32-bit on the device, whatever its tables hold.)
-  if (best_part == 0 || (int64_t)a->num_seqs * a->num_kv_heads * plan.row_tiles * mvr::kPrefillMaxParts >= (1LL << 31)) return;
-  plan.part_steps = (int)best_part;
-  plan.balanced_blocks = (int)blocks_at(best_part);
-  plan.balanced_tiles = (int)tiles;
+  int64_t part_steps = 0;
+  if (!equal)
+    for (int64_t quarters : {1, 2, 3, 4, 8, 12, 16}) { // of a block per CU
+      const int64_t most = std::min(split_override > 1 ? tiles * split_override : quarters * cus / 4, slots);
+      if (most < tiles) continue;
+      int64_t lo = std::min<int64_t>(2, longest), hi = longest; // blocks_at(hi) = tiles <= most
+      while (lo < hi) {
+        const int64_t mid = (lo + hi) / 2;
+        if (blocks_at(mid) <= most)
+          hi = mid;
+        else
+          lo = mid + 1;
+      }
+      if (lo >= longest) continue;
+      int64_t part = 0;
+      const int64_t blocks = blocks_at(lo, &part);
+      const double cost = cost_us(blocks, part, 1.0) + merge_us((blocks + tiles - 1) / tiles) + 3;
+      if (cost < best || split_override > 1) {
+        best = cost;
+        part_steps = lo;
+      }
+      if (split_override > 1) break;
+    }
+  int64_t used = span_tiles * splits;
+  if (part_steps > 0) {
+    // (Part counts are 32-bit on the device, whatever its tables hold.)
+    if ((int64_t)a->num_seqs * a->num_kv_heads * plan.row_tiles * mvr::kPrefillMaxParts >= (1LL << 31)) return;
+    plan.part_steps = (int)part_steps;
+    plan.balanced_blocks = (int)blocks_at(part_steps);
+    plan.balanced_tiles = (int)tiles;
+    used = plan.balanced_blocks;
+  } else if (splits > 1) {
+    plan.kv_splits = (int)splits;
+  } else {
+    return;
+  }
   // Slots for a block per CU at least: up to there the workspace does not
   // depend on the lengths.
-  plan.balanced_slots = (int)std::max<int64_t>(plan.balanced_blocks, std::min(cus, slots));
-  const size_t prow = (size_t)plan.balanced_slots * mvr::kPrefillBlockRows;
+  plan.partial_slots = (int)std::max<int64_t>(used, std::min(cus, slots));
+  const size_t prow = (size_t)plan.partial_slots * mvr::kPrefillBlockRows;
   plan.partial_bytes = align_up(prow * a->head_dim * sizeof(float), 256) + align_up(prow * 2 * sizeof(float), 256);
 }
 
@@ -387,7 +436,8 @@ mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_
       plan.prefill_groups = groups_override;
     else
       plan.prefill_groups = a->dtype == MVR_DTYPE_F16 && live_blocks >= 4LL * device_cus() ? 1 : 2;
-    if (plan.prefill_groups == 2 || a->head_dim > 128) plan_balanced(a, live, n_live, len_live, plan);
+    plan.kv_splits = 1;
+    if (plan.prefill_groups == 2 || a->head_dim > 128) plan_prefill_splits(a, live, n_live, len_live, plan);
     return plan;
   }
   plan.row_blocks = rows_max <= 16 || !all_plans ? 1 : 2;
@@ -662,7 +712,7 @@ int launch_planned(const mvr_paged_attention_args* a, const mvr::PagedAttentionP
     f.out_stride_head = a->out_stride_head;
     f.out_stride_token = a->out_stride_token;
     if (plan.partial_bytes) {
-      const size_t prow = (size_t)plan.balanced_slots * mvr::kPrefillBlockRows;
+      const size_t prow = (size_t)plan.partial_slots * mvr::kPrefillBlockRows;
       char* w = static_cast<char*>(ws);
       f.partial_o = reinterpret_cast<float*>(w);
       f.partial_ml = reinterpret_cast<float*>(w + align_up(prow * a->head_dim * sizeof(float), 256));
@@ -673,6 +723,7 @@ int launch_planned(const mvr_paged_attention_args* a, const mvr::PagedAttentionP
     f.page_size = a->page_size;
     mvr::page_divider(a->page_size, f.page_magic, f.page_magic_shift);
     f.row_tiles = plan.row_tiles;
+    f.kv_splits = plan.kv_splits;
     f.balanced_blocks = plan.balanced_blocks;
     f.part_steps = plan.part_steps;
     f.balanced_tiles = plan.balanced_tiles;
@@ -891,6 +942,7 @@ CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget, bool
   p1 = *a;
   LiveSeqs live1;
   live1.count = count[1];
+  live1.span = last[1] - first[1] + 1;
   live1.prefill_budget = budget;
   if (hinted) use_tables(a, qmax + 1, INT32_MAX, live1);
   if (hinted) {
@@ -902,14 +954,13 @@ CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget, bool
   e1.skip_seq_lo = first[0];
   e1.skip_seq_hi = last[0];
   e1.skip_q_max = qmax;
-  const int span1 = last[1] - first[1] + 1;
-  if (span1 < a->num_seqs && c.plan[1].balanced_blocks == 0) {
+  if (live1.span < a->num_seqs && c.plan[1].balanced_blocks == 0) {
     // Main grid over the prefill range; the rest of the decode range gets a
     // catch-up block per sequence (it exits unless a stale hint put a
     // prefill-sized request there).  (A balanced grid finds every sequence
     // that launch 0 leaves by itself.)
     e1.seq_lo = first[1];
-    e1.seq_count = span1;
+    e1.seq_count = (int32_t)live1.span;
     e1.catch_lo = first[0];
     e1.catch_count = last[0] - first[0] + 1;
   }

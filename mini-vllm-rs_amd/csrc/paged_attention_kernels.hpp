@@ -88,10 +88,11 @@ struct PagedAttentionPlan {
   int64_t num_units;
   size_t partial_bytes; // workspace for partials (0 when max_parts == 1)
   bool prefill;         // chunked-prefill kernel (paged_prefill.hip) instead of the split-context one
-  int balanced_blocks;  // prefill: blocks of the balanced grid (0: a block per row tile),
-  int balanced_slots;   // partial slots (>= balanced_blocks),
+  int kv_splits;        // prefill: parts per row tile of the main grid (1: unsplit)
+  int balanced_blocks;  // prefill: blocks of the balanced grid (0: the main grid),
   int part_steps;       // key steps per part
   int balanced_tiles;   // and row tiles
+  int partial_slots;    // prefill: partial slots of a split grid (>= its parts)
   int prefill_groups;   // prefill: wavefront groups of 4 per block (2, or 1)
   bool block_merge;     // one block per tile, its partitions merged in LDS
   int block_waves;      // block_merge: wavefronts per block, 4, 8 or 16 (>= max_parts)

@@ -29,9 +29,10 @@
 //     from the S^T registers;  O^T += V^T P^T in D/16 MFMAs.
 // Blocks of one (sequence, KV head) are mapped onto one XCD (workgroups are
 // dispatched round-robin over the 8 XCDs), so their shared K/V stays in that
-// XCD's L2.  Grids of few or unequal tiles run balanced instead: each tile's
-// keys in parts of about one length, a block per part, combined by
-// prefill_merge_kernel from an fp32 partial workspace.
+// XCD's L2.  Grids that leave CUs idle split each tile's keys into as many
+// parts (kv_splits), and grids of unequal tiles run balanced, in parts of about
+// one length: a block per part, combined by prefill_merge_kernel from an fp32
+// partial workspace.
 #include "paged_prefill.hpp"
 
 #include <math.h>
@@ -193,13 +194,13 @@ struct Tile {
   __device__ static __forceinline__ int kswz(int t) { return t & (kSwzGroup - 1); }
 };
 
-// Steps [step0, step1) of one (sequence, kv head, 128-row tile); a step is one
-// key tile per group: it stages them, then QK^T, softmax and PV in turn.  Steps
-// past the tile's last visible key are left out.  A part (not all of the
-// tile's steps) writes its unnormalised rows to partial slot `slot`.
+// Key tiles [j0, j_end) of one (sequence, kv head, 128-row tile), in steps of a
+// key tile per group: each stages its tiles, then QK^T, softmax and PV in turn.
+// Tiles past the last that its rows see are left out.  A part (not all of
+// those) writes its unnormalised rows to partial slot `slot`.
 template <int D, typename T, int TT, int G, bool TP>
 __device__ __forceinline__ void prefill_tile_serial(const PrefillParams& p, const SeqRows& s, int b, int h, int rt,
-                                                    int step0, int step1, int slot) {
+                                                    int j0, int j_end, int slot) {
   static_assert(G == 1 || G == 2, "one or two wavefront groups");
   typedef Tile<D, T, TT, G> TL;
   constexpr bool kF32 = TL::kF32;
@@ -231,10 +232,9 @@ __device__ __forceinline__ void prefill_tile_serial(const PrefillParams& p, cons
 
   const int rows = p.group_size * s.q_len;
   const int n_tiles = block_key_tiles<TT>(s, p.group_size, rt);
-  const int j0 = G * step0;
   if (j0 >= n_tiles) return; // whole block: uniform return before any barrier
-  const int j1 = min(G * step1, n_tiles);
-  const bool partial = step0 > 0 || j1 < n_tiles;
+  const int j1 = min(j_end, n_tiles);
+  const bool partial = j0 > 0 || j1 < n_tiles;
 
   // This lane's query row.
   const int rho = rt * kBlockRows + rw * kRowsPerWave + (l & 31);
@@ -953,36 +953,39 @@ __device__ __forceinline__ bool find_part(const PrefillParams& p, int i, PartPos
   }
 }
 
-// Steps of part `part` of a tile in `parts` parts: an even share of the steps
-// that its rows see (fewer parts than that many hold any).
-struct PartSteps {
-  int begin, end, parts; // parts that hold steps
+// Key tiles of part `part` of a row tile in `parts` parts: an even share of
+// those its rows see, in at most as many parts as that makes steps.  (In whole
+// steps: F32 D=64, 98 tiles in 8 parts, 36.9 us against 35.0.)
+struct PartTiles {
+  int begin, end, parts; // parts that hold tiles
 };
 template <int TT, int G>
-__device__ __forceinline__ PartSteps part_steps(const PrefillParams& p, const SeqRows& s, int rt, int parts, int part) {
-  const int own = (block_key_tiles<TT>(s, p.group_size, rt) + G - 1) / G;
-  const int k = min(parts, own);
+__device__ __forceinline__ PartTiles part_tiles(const PrefillParams& p, const SeqRows& s, int rt, int parts, int part) {
+  const int own = block_key_tiles<TT>(s, p.group_size, rt);
+  const int k = min(parts, (own + G - 1) / G);
   if (part >= k) return {0, 0, k};
   const int each = (unsigned)own / (unsigned)k, rest = own - each * k; // the first `rest` parts take one more
   return {part * each + min(part, rest), (part + 1) * each + min(part + 1, rest), k};
 }
 
-// Main grid: block x covers (sequence, kv head, row tile) of the main range,
-// unsplit.  XCD-aware decode: block x runs on XCD x % 8 and all blocks of one
-// (sequence, kv head) pair sit on the same XCD, so their shared K/V stays in
-// that XCD's L2 (with fewer pairs than XCDs, plain linear order keeps every
-// XCD busy).  Catch-up blocks follow the main grid.
+// Main grid: block x covers (sequence, kv head, row tile, part) of the main
+// range, every tile in kv_splits parts (1: unsplit).  XCD-aware decode: block x
+// runs on XCD x % 8 and all blocks of one (sequence, kv head) pair sit on the
+// same XCD, so their shared K/V stays in that XCD's L2 (with fewer pairs than
+// XCDs, plain linear order keeps every XCD busy).  Catch-up blocks follow the
+// main grid.
 __host__ __device__ __forceinline__ int64_t prefill_main_blocks(const PrefillParams& p) {
   const int64_t pairs = (int64_t)(p.seq_count ? p.seq_count : p.num_seqs) * p.num_kv_heads;
-  const int64_t per_pair = p.row_tiles;
+  const int64_t per_pair = (int64_t)p.row_tiles * p.kv_splits;
   return pairs >= kXcds ? kXcds * ((pairs + kXcds - 1) / kXcds) * per_pair : pairs * per_pair;
 }
 
-constexpr int kAllSteps = 1 << 24; // past every tile's last step
+constexpr int kAllTiles = INT32_MAX;
 
 // TP: pages that are not a multiple of 16 tokens, read in place (head_dim 64
-// and 128; the page size a multiple of the tokens one load covers).
-template <int D, typename T, int G, bool TP>
+// and 128; the page size a multiple of the tokens one load covers).  SPLIT:
+// kv_splits > 1 (apart, so that an unsplit block starts without its arithmetic).
+template <int D, typename T, int G, bool TP, bool SPLIT>
 __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) void paged_prefill_kernel(PrefillParams p) {
   constexpr int TT = prefill_tile_tokens<D, T>();
   const int x = blockIdx.x;
@@ -996,12 +999,12 @@ __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) vo
     if (s.q_len <= 0) return;
     for (int h = 0; h < p.num_kv_heads; h++)
       for (int rt = 0; rt < p.row_tiles; rt++) {
-        prefill_tile_serial<D, T, TT, G, TP>(p, s, b, h, rt, 0, kAllSteps, 0);
+        prefill_tile_serial<D, T, TT, G, TP>(p, s, b, h, rt, 0, kAllTiles, 0);
         __syncthreads(); // group 0's hand-off reads end before the next tile refills the stages
       }
     return;
   }
-  const int per_pair = p.row_tiles;
+  const int per_pair = SPLIT ? p.row_tiles * p.kv_splits : p.row_tiles;
   const int pairs = main_seqs * p.num_kv_heads;
   int pair, local;
   if (pairs >= kXcds) {
@@ -1027,16 +1030,26 @@ __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) vo
   // fresh prompts: Llama-3-8B 1 x 2048 F16 75.3 (in order) -> 70.7 (reverse)
   // -> 58.0 us (by position), F32 512.1 -> 480.6 -> 325.9, Qwen2-7B 1 x 8192
   // 667.7 -> 632.6 -> 517.4; chunks on a long prefix level.
-  int rt;
+  int rt, part;
   {
+    const int idx = SPLIT ? (int)((unsigned)local / (unsigned)p.kv_splits) : local;
+    part = SPLIT ? local - idx * p.kv_splits : 0;
     const int tq = s.q_len / kBlockRows; // tiles per query head
     if (s.q_len > 0 && s.q_len % kBlockRows == 0) {
-      rt = local < p.group_size * tq ? (local % p.group_size) * tq + (tq - 1 - local / p.group_size) : local;
+      rt = idx < p.group_size * tq ? (idx % p.group_size) * tq + (tq - 1 - idx / p.group_size) : idx;
     } else {
-      rt = p.row_tiles - 1 - local;
+      rt = p.row_tiles - 1 - idx;
     }
   }
-  prefill_tile_serial<D, T, TT, G, TP>(p, s, b, h, rt, 0, kAllSteps, 0);
+  int j0 = 0, j_end = kAllTiles, slot = 0;
+  if constexpr (SPLIT) {
+    const PartTiles keys = part_tiles<TT, G>(p, s, rt, p.kv_splits, part);
+    if (keys.begin >= keys.end) return;
+    j0 = keys.begin;
+    j_end = keys.end;
+    slot = (((b - p.seq_lo) * p.num_kv_heads + h) * p.row_tiles + rt) * p.kv_splits + part;
+  }
+  prefill_tile_serial<D, T, TT, G, TP>(p, s, b, h, rt, j0, j_end, slot);
 }
 
 // One part of the balanced grid per block (blocks past the last exit; an
@@ -1055,67 +1068,88 @@ __global__ __launch_bounds__(kRowWaves* G * 64, (G == 1 && D <= 128) ? 2 : 1) vo
     PartPos w;
     bool split;
     if (!find_part<Find::kPart, TT, G>(p, i, w, split)) return;
-    const PartSteps steps = part_steps<TT, G>(p, w.s, w.rt, w.parts, w.part);
-    if (steps.begin < steps.end)
-      prefill_tile_serial<D, T, TT, G, TP>(p, w.s, w.b, w.h, w.rt, steps.begin, steps.end,
+    const PartTiles keys = part_tiles<TT, G>(p, w.s, w.rt, w.parts, w.part);
+    if (keys.begin < keys.end)
+      prefill_tile_serial<D, T, TT, G, TP>(p, w.s, w.b, w.h, w.rt, keys.begin, keys.end,
                                            w.slot0 + w.part * seq_row_tiles(p, w.s));
     if (split) return;
     __syncthreads(); // group 0's hand-off reads end before the next tile refills the stages
   }
 }
 
-// Merges the parts of the balanced grid's tiles:
+// Merges the parts of a split grid's tiles:
 //   out = sum_j 2^(m_j - M) o_j / sum_j 2^(m_j - M) l_j,  M = max_j m_j.
 // A wavefront takes the 32 rows of one row wavefront, in the partials' register
 // layout (lane l: row l % 32), and of their dims one float4 per lane (F16: 8
 // consecutive dims of a row) or D / 32 (F32: as many consecutive dims per lane
-// and element).  8 parts (F32: 4), weights and rows, are in flight at once: the
-// kernel is bound by its dependent round trips (lengths, then the parts).
+// and element).  8 parts, weights and rows, are in flight at once: the kernel is
+// bound by its round trips (16 of them took 0.6-1.4 us more, 4 in F32 0.2-1.2).
+// F32 rows of more than 128 elements keep 4, whose 8 spilled.  On the main grid
+// the first parts are requested before the tile's bounds are known, 0.4 us
+// earlier, where registers allow (the slots exist; what those past the tile's
+// parts hold is never used).
 template <int D, bool kF32>
 constexpr int merge_waves_per_tile() {
   return kRowWaves * (kF32 ? 4 : D / 8);
 }
-template <int D, typename T, int G>
+template <int D, typename T, int G, bool BALANCED>
 __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(PrefillParams p) {
   constexpr int TT = prefill_tile_tokens<D, T>();
   constexpr bool kF32 = sizeof(T) == 4;
   constexpr int kVecs = kF32 ? D / 32 : 1; // float4 per lane
-  constexpr int kBatch = kF32 ? 4 : 8;     // parts in flight
+  constexpr int kBatch = kF32 && (BALANCED || D > 128) ? 4 : 8; // parts in flight
+  constexpr bool kEarly = !BALANCED && (!kF32 || D <= 64);
   constexpr int kPerTile = merge_waves_per_tile<D, kF32>();
   static_assert(kPerTile % kMergeWaves == 0, "whole blocks per tile");
-  PartPos t;
-  bool split;
-  if (!find_part<Find::kTile, TT, G>(p, blockIdx.x / (kPerTile / kMergeWaves), t, split) || !split) return;
-  const int parts = part_steps<TT, G>(p, t.s, t.rt, t.parts, 0).parts;
-  if (parts <= 1) return;
-  const int rts = seq_row_tiles(p, t.s);
+  const int tile = blockIdx.x / (kPerTile / kMergeWaves);
   const int l = threadIdx.x & 63;
   const int hh = l >> 5;
   const int unit = blockIdx.x % (kPerTile / kMergeWaves) * kMergeWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rw = unit % kRowWaves, k = unit / kRowWaves; // k: n * 4 + e / 4 (F16) or e / 4 (F32)
-  const int rho = t.rt * kBlockRows + rw * kRowsPerWave + (l & 31);
-  const bool valid = rho < p.group_size * t.s.q_len;
+  // The tile's slots: part j's is slot0 + j * stride, `slots` of them exist.
+  PartPos t;
+  int stride = 1, slots = p.kv_splits;
+  if constexpr (BALANCED) {
+    bool split;
+    if (!find_part<Find::kTile, TT, G>(p, tile, t, split) || !split) return;
+    stride = seq_row_tiles(p, t.s);
+    slots = t.parts;
+  } else {
+    t.rt = tile % p.row_tiles;
+    t.h = tile / p.row_tiles % p.num_kv_heads;
+    t.b = p.seq_lo + tile / (p.row_tiles * p.num_kv_heads);
+    t.slot0 = tile * p.kv_splits;
+  }
   const float2v* ml = reinterpret_cast<const float2v*>(p.partial_ml) + (int64_t)t.slot0 * kBlockRows + rw * kRowsPerWave + (l & 31);
   const float4v* src = reinterpret_cast<const float4v*>(p.partial_o) +
                        ((int64_t)t.slot0 * kRowWaves + rw) * (D / 8 * 64) + k * 64 + l;
+  float2v mlj[kBatch];
+  float4v o[kBatch][kVecs];
+  auto load_batch = [&](int j0, int n) { // (past the n-th part: that one again)
+#pragma unroll
+    for (int u = 0; u < kBatch; u++) {
+      const int64_t j = min(j0 + u, n - 1) * stride;
+      mlj[u] = ml[j * kBlockRows];
+#pragma unroll
+      for (int v = 0; v < kVecs; v++) o[u][v] = src[j * kRowWaves * (D / 8 * 64) + 4 * v * 64];
+    }
+  };
+  if constexpr (kEarly) load_batch(0, slots);
+  if constexpr (!BALANCED) t.s = load_rows(p, t.b);
+  const int parts = part_tiles<TT, G>(p, t.s, t.rt, slots, 0).parts;
+  if (parts <= 1) return;
+  const int rho = t.rt * kBlockRows + rw * kRowsPerWave + (l & 31);
+  const bool valid = rho < p.group_size * t.s.q_len;
   float m = -INFINITY, den = 0.f;
   float4v acc[kVecs];
 #pragma unroll
   for (int v = 0; v < kVecs; v++) acc[v] = float4v{0.f, 0.f, 0.f, 0.f};
   for (int j0 = 0; j0 < parts; j0 += kBatch) {
-    // (Past the last part: its rows again, at weight 0.)
-    float2v mlj[kBatch];
-    float4v o[kBatch][kVecs];
-#pragma unroll
-    for (int u = 0; u < kBatch; u++) {
-      const int64_t j = min(j0 + u, parts - 1) * rts;
-      mlj[u] = ml[j * kBlockRows];
-#pragma unroll
-      for (int v = 0; v < kVecs; v++) o[u][v] = src[j * kRowWaves * (D / 8 * 64) + 4 * v * 64];
-    }
+    if (!kEarly || j0 > 0) load_batch(j0, parts);
     float m_new = m;
 #pragma unroll
-    for (int u = 0; u < kBatch; u++) m_new = fmaxf(m_new, mlj[u][0]);
+    for (int u = 0; u < kBatch; u++)
+      m_new = fmaxf(m_new, kEarly && j0 + u >= parts ? -INFINITY : mlj[u][0]);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const float alpha = __builtin_amdgcn_exp2f(m - m_use); // 0 in the first batch
     den *= alpha;
@@ -1123,12 +1157,13 @@ __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(Prefill
     for (int v = 0; v < kVecs; v++) acc[v] *= alpha;
 #pragma unroll
     for (int u = 0; u < kBatch; u++) {
-      const float w = j0 + u < parts ? __builtin_amdgcn_exp2f(mlj[u][0] - m_use) : 0.f; // m = -inf (no visible key): 0
-      den += w * mlj[u][1];
+      const bool past = j0 + u >= parts, skip = kEarly && past; // skip: it may hold anything
+      const float w = past ? 0.f : __builtin_amdgcn_exp2f(mlj[u][0] - m_use); // m = -inf (no visible key): 0
+      den = skip ? den : den + w * mlj[u][1];
 #pragma unroll
       for (int v = 0; v < kVecs; v++)
 #pragma unroll
-        for (int c = 0; c < 4; c++) acc[v][c] = w == 0.f ? acc[v][c] : fmaf(w, o[u][v][c], acc[v][c]);
+        for (int c = 0; c < 4; c++) acc[v][c] = skip || w == 0.f ? acc[v][c] : fmaf(w, o[u][v][c], acc[v][c]);
     }
     m = m_new;
   }
@@ -1157,24 +1192,32 @@ __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(Prefill
 
 template <int D, typename T, int G, bool TP>
 hipError_t launch_shape(const PrefillParams& params, hipStream_t stream) {
-  if (params.balanced_blocks > 0) {
-    // (One-group blocks up to D=128 are for grids of many blocks per CU.)
-    if constexpr (G == 1 && D <= 128) {
-      return hipErrorInvalidValue;
-    } else {
-      hipLaunchKernelGGL((paged_prefill_balanced_kernel<D, T, G, TP>), dim3((unsigned)params.balanced_blocks),
-                         dim3(kRowWaves * G * 64), 0, stream, params);
+  // (One-group blocks up to D=128 are for grids of many blocks per CU: unsplit.)
+  constexpr bool kSplits = G == 2 || D > 128;
+  const bool balanced = params.balanced_blocks > 0, split = balanced || params.kv_splits > 1;
+  if (params.kv_splits < 1 || (split && !kSplits)) return hipErrorInvalidValue;
+  const dim3 block(kRowWaves * G * 64);
+  const dim3 grid((unsigned)(balanced ? params.balanced_blocks : prefill_main_blocks(params) + params.catch_count));
+  if constexpr (kSplits) {
+    if (split) {
+      if (balanced)
+        hipLaunchKernelGGL((paged_prefill_balanced_kernel<D, T, G, TP>), grid, block, 0, stream, params);
+      else
+        hipLaunchKernelGGL((paged_prefill_kernel<D, T, G, TP, true>), grid, block, 0, stream, params);
       const hipError_t err = hipGetLastError();
       if (err != hipSuccess) return err;
-      hipLaunchKernelGGL((prefill_merge_kernel<D, T, G>),
-                         dim3((unsigned)(params.balanced_tiles * (merge_waves_per_tile<D, sizeof(T) == 4>() / kMergeWaves))),
-                         dim3(64 * kMergeWaves), 0, stream, params);
+      const int64_t tiles = balanced ? params.balanced_tiles
+                                     : (int64_t)(params.seq_count ? params.seq_count : params.num_seqs) *
+                                           params.num_kv_heads * params.row_tiles;
+      const dim3 merge_grid((unsigned)(tiles * (merge_waves_per_tile<D, sizeof(T) == 4>() / kMergeWaves)));
+      if (balanced)
+        hipLaunchKernelGGL((prefill_merge_kernel<D, T, G, true>), merge_grid, dim3(64 * kMergeWaves), 0, stream, params);
+      else
+        hipLaunchKernelGGL((prefill_merge_kernel<D, T, G, false>), merge_grid, dim3(64 * kMergeWaves), 0, stream, params);
+      return hipGetLastError();
     }
-  } else {
-    const int64_t blocks = prefill_main_blocks(params) + params.catch_count;
-    hipLaunchKernelGGL((paged_prefill_kernel<D, T, G, TP>), dim3((unsigned)blocks), dim3(kRowWaves * G * 64), 0,
-                       stream, params);
   }
+  hipLaunchKernelGGL((paged_prefill_kernel<D, T, G, TP, false>), grid, block, 0, stream, params);
   return hipGetLastError();
 }
 

@@ -8,7 +8,7 @@ namespace mvr {
 
 // Rows per block of the prefill kernel (4 wavefronts x 32 grouped rows).
 constexpr int kPrefillBlockRows = 128;
-// Parts per row tile of a balanced grid, at most.
+// Parts per row tile of a split grid, at most.
 constexpr int kPrefillMaxParts = 32;
 
 struct PrefillParams {
@@ -23,8 +23,8 @@ struct PrefillParams {
   int32_t single_seq_len, single_q_len;
   void* out;
   int64_t out_stride_head, out_stride_token;
-  float* partial_o;  // balanced grids: [balanced_blocks][4][head_dim / 8][64] float4, as the registers lie
-  float* partial_ml; // [balanced_blocks][128][2]
+  float* partial_o;  // split grids: [slots][4][head_dim / 8][64] float4, as the registers lie
+  float* partial_ml; // [slots][128][2]
   // page_size: a multiple of 16, or one that prefill_token_pages_supported
   // accepts (read in place by the token-page kernels).
   int32_t num_seqs, num_kv_heads, group_size, page_size;
@@ -33,6 +33,9 @@ struct PrefillParams {
   uint64_t page_magic;
   int32_t page_magic_shift;
   int32_t row_tiles;  // 128-row tiles per (sequence, kv head)
+  // Main grid: parts per row tile (1: unsplit).  Partial slot of (b, h, rt,
+  // part): (((b - seq_lo) * num_kv_heads + h) * row_tiles + rt) * kv_splits + part.
+  int32_t kv_splits;
   // balanced_blocks > 0: a balanced grid of that many blocks in place of the
   // main grid and its catch-up blocks, over every sequence that is not skipped:
   // a block per part of at most part_steps key steps of a row tile (a step is
@@ -48,7 +51,7 @@ struct PrefillParams {
   // Sequences b in [skip_seq_lo, skip_seq_hi] with q_len <= skip_q_max (0:
   // none) belong to another launch of the same call and are skipped.
   int32_t skip_seq_lo, skip_seq_hi, skip_q_max;
-  // Main grid: one block per (sequence, kv head, row tile) for the sequences
+  // Main grid: one block per (sequence, kv head, row tile, part) for the sequences
   // [seq_lo, seq_lo + seq_count) (count 0: every sequence).
   int32_t seq_lo, seq_count;
   // Catch-up blocks after the main grid: one per sequence of [catch_lo,
