@@ -179,13 +179,13 @@ int device_cus() {
 struct LiveSeqs {
   int64_t count = 0;   // sequences with rows in this launch (0: num_seqs)
   int max_seq_len = 0; // their longest context (0: the call's max_seq_len)
-  // Valid host tables of the launch's sequences: those of its num_seqs with
+  // Valid host tables of the launch's sequences: those of its num_seqs (or span) with
   // q_min..q_max new tokens (null: count sequences at the bounds above), the
   // first key_begin keys of each left out.
   const int32_t* cu_q_lens = nullptr;
   const int32_t* seq_lens = nullptr;
   int q_min = 1, q_max = INT32_MAX, key_begin = 0;
-  int64_t span = 0; // prefill kernel: sequences of the main grid (0: num_seqs)
+  int64_t span = 0; // prefill kernel: sequences of the main grid and of the tables (0: num_seqs)
   // Largest workspace a split prefill grid's partials may take.
   size_t prefill_budget = (size_t)48 << 20;
   // The split-context kernel's partials do not fit the workspace given: take
@@ -225,38 +225,49 @@ void plan_prefill_splits(const mvr_paged_attention_args* a, const LiveSeqs& live
   const int64_t cus = device_cus();
   const int group = a->num_q_heads / a->num_kv_heads;
   const int step_keys = prefill_step_keys(a);
-  // fn(tiles, steps per tile) for each sequence of the launch.
-  auto each = [&](auto fn) {
-    if (!live.seq_lens || !live.cu_q_lens) {
-      fn(n_live * a->num_kv_heads * plan.row_tiles, (int64_t)(len_live + step_keys - 1) / step_keys);
-      return;
-    }
-    for (int s = 0; s < a->num_seqs; s++) {
-      const int64_t q = live.cu_q_lens[s + 1] - live.cu_q_lens[s];
-      if (q < live.q_min) continue;
-      fn(a->num_kv_heads * ((group * q + mvr::kPrefillBlockRows - 1) / mvr::kPrefillBlockRows),
-         ((int64_t)live.seq_lens[s] + step_keys - 1) / step_keys);
-    }
+  // The launch's tiles by their number of steps (neighbours of one number
+  // together): planning walks these, not the call's sequences, again and again.
+  struct Tiles {
+    int count, steps;
   };
+  constexpr int kMaxLengths = 256; // on the stack; a call of more keeps the unsplit grid
+  Tiles lengths[kMaxLengths];
+  int n_lengths = 0;
   int64_t tiles = 0, steps = 0, longest = 0;
-  bool equal = true; // sequences of one number of steps
-  each([&](int64_t t, int64_t n) {
-    equal = equal && (tiles == 0 || n == longest);
+  auto add = [&](int64_t t, int n) {
+    if (n_lengths == 0 || lengths[n_lengths - 1].steps != n) {
+      if (n_lengths == kMaxLengths) return false;
+      lengths[n_lengths++] = Tiles{0, n};
+    }
+    lengths[n_lengths - 1].count += (int)t;
     tiles += t;
     steps += t * n;
-    longest = std::max(longest, n);
-  });
-  if (tiles == 0 || tiles > 4 * cus) return;
+    longest = std::max<int64_t>(longest, n);
+    return tiles <= 4 * cus;
+  };
+  if (!live.seq_lens || !live.cu_q_lens) {
+    if (!add(n_live * a->num_kv_heads * plan.row_tiles, (len_live + step_keys - 1) / step_keys)) return;
+  } else {
+    // (A mixed batch's tables begin at the main grid's first sequence.)
+    for (int64_t s = 0; s < (live.span > 0 ? live.span : a->num_seqs); s++) {
+      const int q = live.cu_q_lens[s + 1] - live.cu_q_lens[s];
+      if (q < live.q_min) continue;
+      const int64_t row_tiles = ((int64_t)group * q + mvr::kPrefillBlockRows - 1) / mvr::kPrefillBlockRows;
+      if (!add(a->num_kv_heads * row_tiles, (int)(((int64_t)live.seq_lens[s] + step_keys - 1) / step_keys))) return;
+    }
+  }
+  if (tiles == 0) return;
+  const bool equal = n_lengths == 1; // sequences of one number of steps
   // Blocks of the call in parts of at most `part` steps, and its longest part.
-  auto blocks_at = [&](int64_t part, int64_t* longest_part = nullptr) {
-    int64_t blocks = 0, most = 0;
-    each([&](int64_t t, int64_t n) {
-      const int64_t parts = std::min<int64_t>((n + part - 1) / part, mvr::kPrefillMaxParts);
-      blocks += t * parts;
-      most = std::max(most, (n + parts - 1) / parts);
-    });
+  auto blocks_at = [&](int part, int* longest_part = nullptr) {
+    int blocks = 0, most = 0;
+    for (int i = 0; i < n_lengths; i++) {
+      const int parts = std::min((lengths[i].steps + part - 1) / part, mvr::kPrefillMaxParts);
+      blocks += lengths[i].count * parts;
+      if (longest_part) most = std::max(most, (lengths[i].steps + parts - 1) / parts);
+    }
     if (longest_part) *longest_part = most;
-    return blocks;
+    return (int64_t)blocks;
   };
   const bool f16 = a->dtype == MVR_DTYPE_F16;
   const size_t slot_bytes = (size_t)mvr::kPrefillBlockRows * (a->head_dim + 2) * sizeof(float);
@@ -298,21 +309,23 @@ void plan_prefill_splits(const mvr_paged_attention_args* a, const LiveSeqs& live
       splits = k;
     }
   }
-  int64_t part_steps = 0;
-  if (!equal)
-    for (int64_t quarters : {1, 2, 3, 4, 8, 12, 16}) { // of a block per CU
+  int part_steps = 0;
+  if (!equal) {
+    int shorter = (int)longest; // the last fill's parts: a higher fill's are no longer
+    for (int quarters : {1, 2, 3, 4, 8, 12, 16}) { // of a block per CU
       const int64_t most = std::min(split_override > 1 ? tiles * split_override : quarters * cus / 4, slots);
       if (most < tiles) continue;
-      int64_t lo = std::min<int64_t>(2, longest), hi = longest; // blocks_at(hi) = tiles <= most
+      int lo = (int)std::min<int64_t>(std::max<int64_t>(2, steps / most), shorter), hi = shorter; // blocks_at(hi) <= most
       while (lo < hi) {
-        const int64_t mid = (lo + hi) / 2;
+        const int mid = (lo + hi) / 2;
         if (blocks_at(mid) <= most)
           hi = mid;
         else
           lo = mid + 1;
       }
+      shorter = lo;
       if (lo >= longest) continue;
-      int64_t part = 0;
+      int part = 0;
       const int64_t blocks = blocks_at(lo, &part);
       const double cost = cost_us(blocks, part, 1.0) + merge_us((blocks + tiles - 1) / tiles) + 3;
       if (cost < best || split_override > 1) {
@@ -321,11 +334,12 @@ void plan_prefill_splits(const mvr_paged_attention_args* a, const LiveSeqs& live
       }
       if (split_override > 1) break;
     }
+  }
   int64_t used = span_tiles * splits;
   if (part_steps > 0) {
     // (Part counts are 32-bit on the device, whatever its tables hold.)
     if ((int64_t)a->num_seqs * a->num_kv_heads * plan.row_tiles * mvr::kPrefillMaxParts >= (1LL << 31)) return;
-    plan.part_steps = (int)part_steps;
+    plan.part_steps = part_steps;
     plan.balanced_blocks = (int)blocks_at(part_steps);
     plan.balanced_tiles = (int)tiles;
     used = plan.balanced_blocks;
@@ -381,6 +395,25 @@ bool longest_first_pays(const mvr_paged_attention_args* a, const LiveSeqs& live)
   return load >= 0.7 * std::max({(double)longest, load, (double)last + next});
 }
 
+// Whether the prefill kernel can serve calls of this layout.
+// MVR_ATTN_PREFILL_KERNEL=false keeps every call on the split-context kernel.
+// (Its loads take 16-token runs, 8 in F32, inside one page: page sizes that
+// are multiples of 16, as every size is after the repack; or, at head_dim 64
+// and 128, each load's few whole token rows inside one page: page sizes that
+// prefill_token_pages_supported accepts.)
+bool prefill_kernel_reads(const mvr_paged_attention_args* a) {
+  static const bool enabled = env_bool("MVR_ATTN_PREFILL_KERNEL", true);
+  return enabled && mvr::prefill_head_dim_supported(a->head_dim) &&
+         (a->page_size % mvr::kChunkTokens == 0 ||
+          mvr::prefill_token_pages_supported(a->page_size, a->num_kv_heads, a->head_dim, a->dtype == MVR_DTYPE_F16 ? 2 : 4));
+}
+
+// Many query rows per KV head (chunked prefill): dense contraction, on the
+// LDS-shared 32x32 MFMA kernel (F16 32x32x16, F32 32x32x2).
+bool takes_prefill(const mvr_paged_attention_args* a) {
+  return (int64_t)(a->num_q_heads / a->num_kv_heads) * a->max_q_len > 64 && prefill_kernel_reads(a);
+}
+
 mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_prefill = true,
                                   LiveSeqs live = LiveSeqs{}, bool force_prefill = false) {
   mvr::PagedAttentionPlan plan{};
@@ -396,24 +429,11 @@ mvr::PagedAttentionPlan make_plan(const mvr_paged_attention_args* a, bool allow_
   // decode-sized calls; prefill-sized calls take the prefill kernel as at 64
   // and 128.
   const bool all_plans = mvr::head_dim_all_plans(a->head_dim);
-  // Many query rows per KV head (chunked prefill): dense contraction, use the
-  // LDS-shared 32x32 MFMA kernel (F16 32x32x16, F32 32x32x2).
-  // MVR_ATTN_PREFILL_KERNEL=false keeps every call on the split-context kernel.
-  static const bool prefill_enabled = env_bool("MVR_ATTN_PREFILL_KERNEL", true);
-  // (Its loads take 16-token runs, 8 in F32, inside one page: page sizes
-  // that are multiples of 16, as every size is after the repack; or, at
-  // head_dim 64 and 128, each load's few whole token rows inside one page:
-  // page sizes that prefill_token_pages_supported accepts.)
-  const bool page_runs = a->page_size % mvr::kChunkTokens == 0;
-  const bool prefill_pages =
-      page_runs || mvr::prefill_token_pages_supported(a->page_size, a->num_kv_heads, a->head_dim,
-                                                      a->dtype == MVR_DTYPE_F16 ? 2 : 4);
-  // Other page sizes reach make_plan only for calls that the split-context
-  // kernel serves, which then reads them in place (token pages), or that the
-  // prefill kernel reads in place.
-  plan.token_pages = !page_runs;
-  if (allow_prefill && prefill_enabled && (rows_max > 64 || force_prefill) && prefill_pages &&
-      mvr::prefill_head_dim_supported(a->head_dim)) {
+  // Page sizes that are not multiples of 16 reach make_plan only for calls that
+  // the split-context kernel serves, which then reads them in place (token
+  // pages), or that the prefill kernel reads in place.
+  plan.token_pages = a->page_size % mvr::kChunkTokens != 0;
+  if (allow_prefill && (rows_max > 64 || force_prefill) && prefill_kernel_reads(a)) {
     plan.prefill = true;
     plan.row_tiles = (int)((rows_max + mvr::kPrefillBlockRows - 1) / mvr::kPrefillBlockRows);
     const int64_t live_blocks = n_live * a->num_kv_heads * plan.row_tiles;
@@ -849,21 +869,28 @@ struct CallPlan {
   size_t total = 0;
 };
 
-// budget: the largest workspace of the prefill launch's partials; no_partials:
-// the split-context launch keeps none where it can.
-CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget, bool no_partials = false) {
+// The call as one launch of every sequence.
+CallPlan whole_call(const mvr_paged_attention_args* a, size_t budget, bool no_partials) {
   CallPlan c;
   c.part[0] = *a;
   LiveSeqs all;
   all.prefill_budget = budget;
   all.no_partials = no_partials;
-  use_tables(a, 1, INT32_MAX, all);
+  if (takes_prefill(a) || (a->sum_seq_lens > 0 && a->sum_seq_lens < (int64_t)a->max_seq_len * a->num_seqs))
+    use_tables(a, 1, INT32_MAX, all); // (a uniform decode plan does not read them)
   c.plan[0] = make_plan(a, true, all);
   c.total = c.plan[0].partial_bytes;
+  return c;
+}
+
+// budget: the largest workspace of the prefill launch's partials; no_partials:
+// the split-context launch keeps none where it can.
+CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget, bool no_partials = false) {
+  CallPlan c;
   const int group = a->num_q_heads / a->num_kv_heads;
   const int small_q = kSmallRows / group; // largest q_len of the small class (0: no such class)
-  if (a->num_seqs < 2 || small_q < 1 || a->max_q_len <= small_q) return c;
-  if (!c.plan[0].prefill) return c; // launch 1 needs the prefill kernel
+  // (Launch 1 needs the prefill kernel.)
+  if (a->num_seqs < 2 || small_q < 1 || a->max_q_len <= small_q || !takes_prefill(a)) return whole_call(a, budget, no_partials);
   const int32_t* cu = a->cu_q_lens_host;
   const int32_t* sl = a->seq_lens_host;
   int first[2] = {-1, -1}, last[2] = {-1, -1}, count[2] = {0, 0}, lmax[2] = {0, 0}, qmax = 0;
@@ -886,7 +913,7 @@ CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget, bool
     lsum[k] += L;
     if (L > lmax[k]) lmax[k] = L;
   }
-  if (hinted && (count[0] == 0 || count[1] == 0)) return c; // one class: one unfiltered launch
+  if (hinted && (count[0] == 0 || count[1] == 0)) return whole_call(a, budget, no_partials); // one class: one unfiltered launch
   if (!hinted) {
     // Without hints the small class is the decode shape, up to 16 grouped
     // rows (one 16-row tile, the block-merge plans); longer queries,
@@ -902,7 +929,7 @@ CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget, bool
     // Unknown total_q: one prefill request.
     const int64_t excess = a->total_q > 0 ? (int64_t)a->total_q - a->num_seqs : 0;
     int64_t n_pref = excess > 0 ? (excess + a->max_q_len - 2) / (a->max_q_len - 1) : 1;
-    if (n_pref >= a->num_seqs) return c;
+    if (n_pref >= a->num_seqs) return whole_call(a, budget, no_partials);
     count[0] = a->num_seqs - (int)n_pref;
     count[1] = (int)n_pref;
     first[0] = 0;
@@ -927,10 +954,10 @@ CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget, bool
   live0.no_partials = no_partials;
   if (hinted) {
     if (sl) live0.max_seq_len = lmax[0];
-    use_tables(a, 1, qmax, live0);
-    if (live0.seq_lens) {
-      live0.cu_q_lens += f;
-      live0.seq_lens += f;
+    if (sl) { // (both tables: within the call's bounds, above)
+      live0.cu_q_lens = cu + f;
+      live0.seq_lens = sl + f;
+      live0.q_max = qmax;
     }
     p0.sum_seq_lens = sl ? lsum[0] : 0; // this class's keys (a speed hint)
   }
@@ -944,9 +971,13 @@ CallPlan plan_call_within(const mvr_paged_attention_args* a, size_t budget, bool
   live1.count = count[1];
   live1.span = last[1] - first[1] + 1;
   live1.prefill_budget = budget;
-  if (hinted) use_tables(a, qmax + 1, INT32_MAX, live1);
   if (hinted) {
-    if (sl) live1.max_seq_len = lmax[1];
+    if (sl) {
+      live1.max_seq_len = lmax[1];
+      live1.cu_q_lens = cu + first[1];
+      live1.seq_lens = sl + first[1];
+      live1.q_min = qmax + 1;
+    }
     p1.sum_seq_lens = sl ? lsum[1] : 0;
   }
   c.plan[1] = make_plan(&p1, true, live1, /*force_prefill=*/true);
@@ -1027,10 +1058,7 @@ bool needs_repack(const mvr_paged_attention_args* a) {
     return false;
   mvr_paged_attention_args b = *a;
   b.page_size = mvr::kChunkTokens; // the plan the repacked call would take
-  const CallPlan c = make_call_plan(&b);
-  for (int k = 0; k < c.n; k++)
-    if (c.plan[k].prefill) return true;
-  return false;
+  return takes_prefill(&b);
 }
 
 RepackPlan make_repack_plan(const mvr_paged_attention_args* a, char* ws, size_t limit = SIZE_MAX) {
