@@ -1,5 +1,5 @@
 """GPU parity of the prefill kernel's main grid with every row tile's keys in the same number of parts (sequences of one
-length, or no host tables): parts found from the block index, merged from fp32 partials.
+length, few unequal ones, or no host tables): parts found from the block index, merged from fp32 partials.
 
 Cases at the places where parts can go wrong: one key tile more or less than a whole number of parts, parts of less
 than a step, up to 32 parts (several rounds of the merge's 8, and of the 4 that wide F32 rows keep), fresh prompts whose
@@ -48,6 +48,15 @@ CASES = {
     "f16 no workspace": ("f16", 28, 4, 128, 16, [100], [4289], "yes", 0),
     "f16 chunks among decodes": ("f16", 32, 8, 128, 16, [1, 130, 1, 1, 130, 1], [90, 2000, 700, 5, 2000, 300], "yes", 1),
     "f16 chunk among decodes, no tables": ("f16", 32, 8, 128, 16, [1, 130, 1, 1], [90, 2000, 700, 5], "no", 1),
+    "f16 130 on 4000": ("f16", 32, 8, 128, 16, [130], [4000], "yes", 1),
+    "f16 17 on 1500": ("f16", 8, 2, 128, 16, [17], [1500], "yes", 1),
+    "f16 chunk behind 70 decodes": ("f16", 32, 8, 128, 16, [1] * 70 + [129], [200] * 70 + [3000], "yes", 1),
+    "f16 chunk before 70 decodes, no tables": ("f16", 32, 8, 128, 16, [129] + [1] * 70, [3000] + [200] * 70, "no", 1),
+    "f16 d64 unequal, token pages": ("f16", 14, 2, 64, 24, [40, 200, 97], [3000, 7000, 4100], "yes", 1),
+    "f32 d64 unequal, 4-token pages": ("f32", 14, 2, 64, 4, [41, 77], [1000, 3100], "yes", 1),
+    "f16 d256 unequal": ("f16", 8, 2, 256, 16, [100, 33], [2500, 900], "yes", 1),
+    "f32 d96 unequal": ("f32", 8, 2, 96, 16, [100, 33], [2500, 900], "yes", 1),
+    "f32 unequal, no tables": ("f32", 28, 4, 128, 16, [117] * 3, [1860, 2320, 897], "no", 1),
     "f16 d64": ("f16", 14, 2, 64, 16, [256], [2048], "yes", 1),
     "f16 d64 token pages": ("f16", 14, 2, 64, 24, [97] * 2, [3000] * 2, "yes", 1),
     "f16 d128 4-token pages": ("f16", 8, 2, 128, 4, [70], [3001], "yes", 1),
