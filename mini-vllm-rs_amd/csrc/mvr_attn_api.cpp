@@ -694,7 +694,7 @@ namespace {
 struct LaunchExtras {
   int32_t class_q_min = 0, class_q_max = 0; // split-context kernel: sequences outside [min, max] (max 0: unbounded) are skipped
   // Prefill kernel: sequences in [skip_seq_lo, skip_seq_hi] with q_len <= skip_q_max (0: none) are skipped;
-  // the main grid (key splits included) covers [seq_lo, seq_lo + seq_count) (count 0: all), and one
+  // the main grid covers [seq_lo, seq_lo + seq_count) (count 0: all), in kv_splits parts per row tile, and one
   // catch-up block per sequence of [catch_lo, catch_lo + catch_count) outside it computes that sequence unsplit.
   int32_t skip_seq_lo = 0, skip_seq_hi = -1, skip_q_max = 0;
   int32_t seq_lo = 0, seq_count = 0, catch_lo = 0, catch_count = 0;

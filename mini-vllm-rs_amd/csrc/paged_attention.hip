@@ -22,6 +22,7 @@
 // flight per wavefront; three for the plans that ask for a deep pipeline).  Partitions of one (b, h, rt) are merged by
 // merge_partitions_kernel with the usual max / sum-of-exponentials rescale.
 #include "paged_attention_kernels.hpp"
+#include "wave_scan.hpp"
 
 #include <math.h>
 
@@ -111,18 +112,6 @@ __device__ __forceinline__ int tile_chunks(const SeqInfo& s, int group_size, int
 __device__ __forceinline__ int tile_parts(const PagedAttentionParams& p, const SeqInfo& s, int n_chunks) {
   const int kb = s.key_begin / kChunkTokens;
   return n_chunks > kb ? min((n_chunks - kb + p.chunks_per_part - 1) / p.chunks_per_part, p.max_parts) : 0;
-}
-
-// Inclusive prefix sum over the 64 lanes of a wavefront: rows of 16 by shifts,
-// then each row's last lane into the rows after it (DPP, no LDS round trips).
-__device__ __forceinline__ int wave_inclusive_sum(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false); // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false); // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false); // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false); // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false); // row_bcast:15 into rows 1 and 3
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false); // row_bcast:31 into rows 2 and 3
-  return v;
 }
 
 // Dense layout of a ragged batch (one row tile per sequence and KV head):
@@ -412,10 +401,12 @@ struct F32Traits {
 // and no merge launch (which costs about 8 us of launch gap and kernel time
 // whatever its work).  The planner uses it when a uniform batch splits every
 // context into more than WPB / 2 and at most WPB partitions, WPB = 4, 8 or
-// 16 (the wavefronts of a block then do near-equal work); a partition
-// without keys still takes part in the block's barriers.
-// DENSE: the dense layout of a ragged batch (dense_unit); a separate instantiation,
-// so that the slot == partition kernels compile exactly as without it.
+// 16 (the wavefronts of a block then do near-equal work), and, with DENSE, for
+// ragged batches of one-tile sequences, longest first; a partition without
+// keys still takes part in the block's barriers.
+// DENSE: the dense layout of a ragged batch (dense_unit; with BM the ranked
+// order of ranked_seq); a separate instantiation, so that the slot == partition
+// kernels compile exactly as without it.
 // DEPTH: chunks in flight per wavefront.  3 (deep_pipeline plans: 16-row
 // tiles whose K and V chunk take 32 VGPRs per lane) costs 192-208 VGPRs, so two
 // wavefronts per SIMD instead of three; that pays on ragged batches of few
@@ -1027,12 +1018,10 @@ hipError_t launch_typed(const PagedAttentionPlan& plan, const PagedAttentionPara
         } else {
           return hipErrorInvalidValue;
         }
-      } else if (plan.dense_parts) { // longest first
-        if (params.row_tiles != 1) return hipErrorInvalidValue;
-        if (plan.block_waves == 4) {
-          hipLaunchKernelGGL((paged_attention_kernel<Tr, D, NB, true, true, 2, 4>), dim3((unsigned)tiles),
-                             dim3(kWaveSize * 4), 0, stream, params);
-        } else if (plan.block_waves == 8) {
+      } else if (plan.dense_parts) {
+        // Longest first: 8-wavefront blocks, rows of at least 256 bytes.
+        if constexpr (D * sizeof(typename Tr::elem) >= 256) {
+          if (params.row_tiles != 1 || plan.block_waves != 8) return hipErrorInvalidValue;
           hipLaunchKernelGGL((paged_attention_kernel<Tr, D, NB, true, true, 2, 8>), dim3((unsigned)tiles),
                              dim3(kWaveSize * 8), 0, stream, params);
         } else {

@@ -96,7 +96,7 @@ struct PagedAttentionPlan {
   int prefill_groups;   // prefill: wavefront groups of 4 per block (2, or 1)
   bool block_merge;     // one block per tile, its partitions merged in LDS
   int block_waves;      // block_merge: wavefronts per block, 4, 8 or 16 (>= max_parts)
-  bool dense_parts;     // ragged split plan: live units first, in a dense order (see dense_unit)
+  bool dense_parts;     // ragged plan: live units first, in a dense order (dense_unit); with block_merge longest first
   bool deep_pipeline;   // three chunks in flight per wavefront instead of two (16-row tiles only)
   int unit_waves;       // split plans without block merge: wavefronts per block, 1, 2 or 4 (0 means 4)
   bool token_pages;     // pages that do not hold whole 16-token chunks, read in place (page_size >= 2)

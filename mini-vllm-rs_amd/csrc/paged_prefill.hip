@@ -34,6 +34,7 @@
 // one length: a block per part, combined by prefill_merge_kernel from an fp32
 // partial workspace.
 #include "paged_prefill.hpp"
+#include "wave_scan.hpp"
 
 #include <math.h>
 
@@ -861,18 +862,6 @@ constexpr int prefill_tile_tokens() {
 // give most blocks two tiles, and a tile costs about 9 us beside its steps:
 // 34 against 24 us on a 256-token chunk behind 2,048 tokens, F16, and 173
 // against 167 us on three ragged F32 chunks.)
-
-// Inclusive sum over the wavefront's lanes: rows of 16 by shifts, then each
-// row's last lane into the rows after it (DPP, no LDS round trips).
-__device__ __forceinline__ int wave_inclusive_sum(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false); // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false); // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false); // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false); // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false); // row_bcast:15 into rows 1 and 3
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false); // row_bcast:31 into rows 2 and 3
-  return v;
-}
 
 __device__ __forceinline__ int seq_row_tiles(const PrefillParams& p, const SeqRows& s) {
   return min((p.group_size * s.q_len + kBlockRows - 1) / kBlockRows, p.row_tiles);
