@@ -26,7 +26,7 @@ MFMA_F32_PEAK_TFLOPS = 157.3   # MI355X dense fp32 MFMA
 # SHA-256 of TRAFFIC_SOURCES concatenated): after any change to them the figure is stale and not reported.
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "paged_attention_decode_b64_ctx8192_f16_hbm_traffic.md")
 TRAFFIC_SOURCES = [os.path.join(ROOT, "mini-vllm-rs_amd", "csrc", f)
-                   for f in ("paged_attention.hip", "paged_attention_kernels.hpp")]
+                   for f in ("paged_attention.hip", "paged_attention_kernels.hpp", "wave_scan.hpp")]
 
 
 def traffic_source_sha256():
