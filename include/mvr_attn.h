@@ -132,11 +132,13 @@ typedef struct mvr_paged_attention_args {
 /* Bytes of workspace mvr_paged_attention needs for these arguments (depends
    on the scalar fields and the planning hints; 0 when no sequence is split
    into context partitions and page_size is a multiple of 16).  Host tables of
-   other contents may need more for the plan that suits them, but no call is
-   refused for that: with less, a prefill launch splits its keys as far as the
-   workspace it is given allows, down to not at all, and a ragged decode merges
-   every sequence's partitions inside one block.  A workspace sized without the
-   host tables holds a decode call's plan for any tables.  The workspace holds fp32
+   other contents may want more for the plan that suits them.  With less, a
+   prefill launch splits its keys as far as the workspace it is given allows,
+   down to not at all, and a ragged decode (pages of 16-token multiples, head
+   rows of at least 256 bytes: where the tables choose between plans) merges
+   every sequence's partitions inside one block; so a decode call is not refused
+   for tables that differ from those it was sized with, and sized without host
+   tables it has what any of them want.  The workspace holds fp32
    partial results of the partitions and, when page_size is not a multiple of
    16, a copy of the batch's K/V in 16-token pages (num_seqs x
    ceil(max_seq_len / 16) pages) with its block table; its contents need no
