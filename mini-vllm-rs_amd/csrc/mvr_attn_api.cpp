@@ -230,7 +230,7 @@ void plan_prefill_splits(const mvr_paged_attention_args* a, const LiveSeqs& live
   struct Tiles {
     int count, steps;
   };
-  constexpr int kMaxLengths = 256; // on the stack; a call of more keeps the unsplit grid
+  constexpr int kMaxLengths = 1024; // on the stack: as many as a call of 4 tiles per CU can have
   Tiles lengths[kMaxLengths];
   int n_lengths = 0;
   int64_t tiles = 0, steps = 0, longest = 0;
@@ -246,7 +246,7 @@ void plan_prefill_splits(const mvr_paged_attention_args* a, const LiveSeqs& live
     return tiles <= 4 * cus;
   };
   if (!live.seq_lens || !live.cu_q_lens) {
-    if (!add(n_live * a->num_kv_heads * plan.row_tiles, (len_live + step_keys - 1) / step_keys)) return;
+    if (!add(n_live * a->num_kv_heads * plan.row_tiles, (int)(((int64_t)len_live + step_keys - 1) / step_keys))) return;
   } else {
     // (A mixed batch's tables begin at the main grid's first sequence.)
     for (int64_t s = 0; s < (live.span > 0 ? live.span : a->num_seqs); s++) {

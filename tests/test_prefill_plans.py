@@ -107,3 +107,11 @@ def test_balanced(plan, name):
         assert parts.max() > 4 and parts.max() % 4, (p, parts)
     if "past 8" in name:
         assert parts.max() > 8 and parts.max() % 8, (p, parts)
+
+
+def test_many_lengths(plan):
+    """As many different lengths as a splittable call can have (4 row tiles per CU) are all planned."""
+    n = 500
+    seq = 300 + 130 * (np.arange(n) % 40) + 4000 * (np.arange(n) % 37 == 0)
+    p = plan("f32", 4, 1, 128, 16, 30, int(seq.max()), True, [30] * n, seq)
+    assert p["blocks"] > n, p
