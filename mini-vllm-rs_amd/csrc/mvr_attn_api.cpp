@@ -202,120 +202,166 @@ int prefill_step_keys(const mvr_paged_attention_args* a) {
 // Split prefill grids, where the unsplit one, a block per row tile, leaves CUs
 // idle or waits for its longest sequence: each tile's keys in parts, a block
 // per part, and a merge launch.  Either every tile of the main grid in kv_splits
-// parts, whose blocks and merge find theirs from the block index, or, for
-// sequences of unequal lengths, the balanced grid's parts of at most part_steps
-// steps, found by a scan of the length tables.  Both are priced, the balanced
-// grid for one to four rounds of blocks over the CUs and for fewer parts that
-// leave CUs idle (the shortest parts whose blocks fit).
-// Measured (one box, HIP events, 47 calls of one length, each in 1..32 parts;
-// F16 and F32, D=64..256, 17..1,024 new tokens on 0..16,000): a step of the
-// two-group block takes 1.45 us in F16 at D=128 (0.57 of that at D=64: its
-// softmax does not shrink), 0.85 us more with every CU busy, and 7.7 / 0.65 us
-// in F32; a block costs 7.2 us beside its steps; the merge launch 4 us, 1.5 us
-// more from 64 tiles on and 2.5 us per 8 parts after the first 8; the balanced
-// grid's scans 3 us more.  The parts chosen so took 0.9% longer than the best on
-// average, at most 5% (one case of 13% at D=256).  F16, 256 tokens on 2,048, 64
-// tiles: 35.4 us unsplit, 29.3 / 26.4 / 26.4 / 35.6 in 2 / 3 / 4 / 5 parts; 64
-// on 8,128, 16 tiles: 102.6, and 36.4 / 25.9 / 24.4 / 33.1 in 4 / 8 / 16 / 20;
-// D=64, 2 x 153 on 600, 80 tiles: 13.3, 16.8 in 2; F32, 256 on 2,048, 56 tiles:
-// 278, 87.1 / 130 in 4 / 5; 3 x 217 on 897..2,320: 309, 168 in parts of at most
-// 20 steps.
+// parts, whose blocks and merge find theirs from the block index, or the
+// balanced grid's parts of at most part_steps steps, found by a scan of the
+// length tables.  Every part count of the first is priced, and of the second the
+// shortest parts whose blocks fit one to four rounds over the CUs, or leave some
+// idle.
+// Measured (one box, HIP events, 127 calls in up to 32 parts: F16 and F32, D=64
+// to 256, 1 to 6 sequences of one or of several lengths, 17..1,500 new tokens on
+// 0..16,000): a step of the two-group block takes 1.45 us in F16 at D=128 (0.57
+// of that at D=64: its softmax does not shrink) and 7.7 us in F32, 0.8 / 0.5 us
+// more with every CU busy; a block costs 7.2 us beside its steps, 0.9 more with
+// every CU busy; a merge launch 3.7 us, 1.5 more from 64 tiles on, 2.2 per 8
+// parts after the first 8 and 5.8 per CU-full of partial rows after the first
+// (at D=128; up to there they stay in the caches); the balanced grid's scans 3
+// us.  The parts chosen so took 0.7% longer than the best on average.  F16, 256
+// tokens on 2,048, 64 tiles: 35.4 us unsplit, 29.3 / 26.4 / 26.4 / 35.6 in 2 / 3
+// / 4 / 5 parts; 64 on 8,128, 16 tiles: 102.6, and 36.4 / 25.9 / 24.4 / 33.1 in 4
+// / 8 / 16 / 20; 5 x 300 on 2,000, 340 tiles: 77.8, 115 in 2; F32, 256 on 2,048,
+// 56 tiles: 278, 87.1 / 130 in 4 / 5; 3 x 217 on 897..2,320: 309, 168 in parts
+// of at most 20 steps.
 void plan_prefill_splits(const mvr_paged_attention_args* a, const LiveSeqs& live, int64_t n_live, int len_live,
                          mvr::PagedAttentionPlan& plan) {
   const int64_t cus = device_cus();
   const int group = a->num_q_heads / a->num_kv_heads;
+  const int groups = a->head_dim > 128 ? 1 : 2; // key tiles per step
   const int step_keys = prefill_step_keys(a);
   // The launch's tiles by their number of steps (neighbours of one number
   // together): planning walks these, not the call's sequences, again and again.
   struct Tiles {
     int count, steps;
+    double work; // steps that their rows see, on average: rows of one head see up to their own position
   };
   constexpr int kMaxLengths = 1024; // on the stack: as many as a call of 4 tiles per CU can have
   Tiles lengths[kMaxLengths];
   int n_lengths = 0;
-  int64_t tiles = 0, steps = 0, longest = 0;
-  auto add = [&](int64_t t, int n) {
-    if (n_lengths == 0 || lengths[n_lengths - 1].steps != n) {
-      if (n_lengths == kMaxLengths) return false;
-      lengths[n_lengths++] = Tiles{0, n};
+  int64_t tiles = 0, longest = 0; // longest: key tiles
+  int last = 0;                   // steps of the launch's last sequence
+  double work = 0;
+  // `count` sequences of q new tokens and n in all.
+  auto add = [&](int64_t count, int64_t q, int64_t n) -> double {
+    const int64_t t = count * a->num_kv_heads * ((group * q + mvr::kPrefillBlockRows - 1) / mvr::kPrefillBlockRows);
+    const double seen = (n - std::max<int64_t>(0, q - mvr::kPrefillBlockRows) / 2.0) / step_keys;
+    last = (int)((n + step_keys - 1) / step_keys);
+    tiles += t;
+    if (tiles > 4 * cus) return -1;
+    if (n_lengths == 0 || lengths[n_lengths - 1].steps != last) {
+      if (n_lengths == kMaxLengths) return -1;
+      lengths[n_lengths++] = Tiles{0, last, 0};
     }
     lengths[n_lengths - 1].count += (int)t;
-    tiles += t;
-    steps += t * n;
-    longest = std::max<int64_t>(longest, n);
-    return tiles <= 4 * cus;
+    lengths[n_lengths - 1].work += t * seen;
+    work += t * seen;
+    longest = std::max(longest, (n * groups + step_keys - 1) / step_keys);
+    return t * seen;
   };
+  // The main grid deals whole (sequence, KV head) pairs to the 8 XCDs, where
+  // there are 8: share is the busiest one's work over an even share (3 x 50 F16
+  // tokens on 3,000 are 12 pairs, two on four of the XCDs: 24.1 us in 5 parts,
+  // 35.0 in 6, whose 36 blocks there need a second round).
+  const int64_t span = live.span > 0 && live.span < a->num_seqs ? live.span : a->num_seqs;
+  const int64_t pairs = span * a->num_kv_heads;
+  double share = 1;
   if (!live.seq_lens || !live.cu_q_lens) {
-    if (!add(n_live * a->num_kv_heads * plan.row_tiles, (int)(((int64_t)len_live + step_keys - 1) / step_keys))) return;
+    if (add(n_live, a->max_q_len, len_live) < 0) return;
+    if (n_live == span && pairs >= 8) share = 8.0 * ((pairs + 7) / 8) / pairs;
   } else {
     // (A mixed batch's tables begin at the main grid's first sequence.)
-    for (int64_t s = 0; s < (live.span > 0 ? live.span : a->num_seqs); s++) {
+    double xcd[8] = {};
+    for (int64_t s = 0; s < span; s++) {
       const int q = live.cu_q_lens[s + 1] - live.cu_q_lens[s];
       if (q < live.q_min) continue;
-      const int64_t row_tiles = ((int64_t)group * q + mvr::kPrefillBlockRows - 1) / mvr::kPrefillBlockRows;
-      if (!add(a->num_kv_heads * row_tiles, (int)(((int64_t)live.seq_lens[s] + step_keys - 1) / step_keys))) return;
+      const double seq_work = add(1, q, live.seq_lens[s]);
+      if (seq_work < 0) return;
+      for (int h = 0; h < std::min(a->num_kv_heads, 8); h++) // (more heads than XCDs: dealt evenly enough)
+        xcd[(s * a->num_kv_heads + h) & 7] += seq_work;
     }
+    double sum = 0;
+    for (double w : xcd) sum += w;
+    if (pairs >= 8 && sum > 0) share = 8 * *std::max_element(xcd, xcd + 8) / sum;
   }
   if (tiles == 0) return;
-  const bool equal = n_lengths == 1; // sequences of one number of steps
-  // Blocks of the call in parts of at most `part` steps, and its longest part.
-  auto blocks_at = [&](int part, int* longest_part = nullptr) {
-    int blocks = 0, most = 0;
-    for (int i = 0; i < n_lengths; i++) {
-      const int parts = std::min((lengths[i].steps + part - 1) / part, mvr::kPrefillMaxParts);
-      blocks += lengths[i].count * parts;
-      if (longest_part) most = std::max(most, (lengths[i].steps + parts - 1) / parts);
-    }
-    if (longest_part) *longest_part = most;
-    return (int64_t)blocks;
-  };
-  const bool f16 = a->dtype == MVR_DTYPE_F16;
   const size_t slot_bytes = (size_t)mvr::kPrefillBlockRows * (a->head_dim + 2) * sizeof(float);
   const int64_t slots = (int64_t)(live.prefill_budget / slot_bytes);
   const double dims = a->head_dim / 128.0;
-  // `blocks` of at most `part` steps; `share`: the busiest XCD's blocks over an
-  // even share of them.
-  auto cost_us = [&](int64_t blocks, double part, double share) {
+  // `blocks` of at most `part` steps, the busiest XCD `busiest` times an even
+  // share; `tail`: steps that the last ones run alone.
+  auto cost_us = [&](int64_t blocks, double part, double busiest, double tail) {
     const double fill = std::min(1.0, (double)blocks / cus);
-    const double step = f16 ? (1.45 + 0.85 * fill) * (0.13 + 0.87 * dims) : (7.7 + 0.65 * fill) * dims;
-    const double busy = blocks * share;
-    const double load = busy <= cus ? part : std::max(part, share * steps / cus + part / 2);
-    return load * step + 7.2 * ceil(busy / cus);
+    const double step = a->dtype == MVR_DTYPE_F16 ? (1.45 + 0.8 * fill) * (0.13 + 0.87 * dims) : (7.7 + 0.5 * fill) * dims;
+    double rounds = blocks * busiest / cus, load = part;
+    if (rounds > 1) {
+      load = std::min(ceil(rounds) * part, std::max(part, busiest * work / cus + tail));
+      rounds = std::min(ceil(rounds), rounds + 0.33);
+    } else {
+      rounds = 1;
+    }
+    return load * step + (7.2 + 0.9 * fill) * rounds;
   };
-  auto merge_us = [&](int64_t parts) {
-    return 4.0 + 1.5 * std::min(1.0, tiles / 64.0) + 2.5 * ((parts - 1) / 8);
+  auto merge_us = [&](int64_t blocks) {
+    const int64_t parts = (blocks + tiles - 1) / tiles;
+    return 3.7 + 1.5 * std::min(1.0, tiles / 64.0) + 2.2 * ((parts - 1) / 8) +
+           5.8 * std::max(0.0, (double)blocks / cus - 1) * dims;
   };
-  // The main grid deals whole (sequence, KV head) pairs to the 8 XCDs: 12 pairs
-  // put two on four of them (3 x 50 F16 tokens on 3,000, 36 tiles: 24.1 us in 5
-  // parts, 35.0 in 6, whose 36 blocks per XCD need a second round).
-  const int64_t span = live.span > 0 && live.span < a->num_seqs ? live.span : a->num_seqs;
-  const int64_t span_tiles = span * a->num_kv_heads * plan.row_tiles;
-  const int64_t pairs = span * a->num_kv_heads;
-  const double share = tiles == span_tiles && pairs >= 8 ? 8.0 * ((pairs + 7) / 8) / pairs : 1.0;
   static const int split_override = env_int("MVR_ATTN_PREFILL_SPLITS", 0);
   if (split_override == 1) return;
-  double best = split_override > 1 ? INFINITY : cost_us(tiles, longest, share);
-  // As many parts for every tile: up to a block per CU, or any number of rounds
-  // for sequences of one length.
-  const int64_t most_parts = std::min<int64_t>(
-      {longest, (int64_t)mvr::kPrefillMaxParts, slots / span_tiles, (equal ? 4 : 1) * cus / tiles,
-       split_override > 1 ? split_override : INT32_MAX});
-  const int64_t groups = a->head_dim > 128 ? 1 : 2; // key tiles per step: its parts end at any tile
+  const bool equal = n_lengths == 1; // sequences of one number of steps
+  double best = split_override > 1 ? INFINITY : cost_us(tiles, (double)longest / groups, share, 0.5 * last);
+  // As many parts for every tile: of unequal sequences up to a block per CU (6 x
+  // 119 F16 tokens on 1,695..3,645, 144 tiles: 58 us unsplit, 65 in 2 parts).
+  const int64_t span_tiles = pairs * plan.row_tiles;
+  const int64_t most_parts =
+      std::min<int64_t>({(longest + groups - 1) / groups, (int64_t)mvr::kPrefillMaxParts, slots / span_tiles,
+                         (equal ? 4 : 1) * cus / tiles, split_override > 1 ? split_override : INT32_MAX});
   int64_t splits = 1;
   for (int64_t k = split_override > 1 ? most_parts : 2; k <= most_parts && k > 1; k++) {
-    const double cost = cost_us(tiles * k, (double)((longest * groups + k - 1) / k) / groups, share) + merge_us(k);
+    const double cost =
+        cost_us(tiles * k, (double)((longest + k - 1) / k) / groups, share, 0.5 * last / k) + merge_us(tiles * k);
     if (cost < best) {
       best = cost;
       splits = k;
     }
   }
+  // Parts of at most part_steps steps.
+  struct Parts {
+    int blocks, longest;
+    double busiest; // of the XCDs, which take an eighth of the blocks each, in order
+  };
+  auto blocks_at = [&](int part) {
+    int blocks = 0;
+    for (int i = 0; i < n_lengths; i++)
+      blocks += lengths[i].count * std::min((lengths[i].steps + part - 1) / part, mvr::kPrefillMaxParts);
+    return blocks;
+  };
+  auto parts_at = [&](int part) {
+    Parts r{blocks_at(part), 0, 1};
+    double xcd[8] = {}, at = 0;
+    const double each = r.blocks / 8.0;
+    for (int i = 0; i < n_lengths; i++) {
+      const int parts = std::min((lengths[i].steps + part - 1) / part, mvr::kPrefillMaxParts);
+      r.longest = std::max(r.longest, (lengths[i].steps + parts - 1) / parts);
+      double left = (double)lengths[i].count * parts;
+      const double per_block = lengths[i].work / left;
+      while (left > 1e-6) {
+        const int x = std::min(7, (int)((at + 1e-6) / each));
+        const double n = x == 7 ? left : std::min(left, std::max((x + 1) * each - at, 1e-3));
+        xcd[x] += n * per_block;
+        at += n;
+        left -= n;
+      }
+    }
+    if (r.blocks > cus && r.blocks % 8 == 0) r.busiest = 8 * *std::max_element(xcd, xcd + 8) / work;
+    return r;
+  };
   int part_steps = 0;
-  if (!equal) {
-    int shorter = (int)longest; // the last fill's parts: a higher fill's are no longer
+  if (!equal || (share > 1.0 && split_override <= 1)) { // (else the main grid's parts are the same, without the scans)
+    const int most_steps = (int)((longest + groups - 1) / groups);
+    int shorter = most_steps; // the last fill's parts: a higher fill's are no longer
     for (int quarters : {1, 2, 3, 4, 8, 12, 16}) { // of a block per CU
       const int64_t most = std::min(split_override > 1 ? tiles * split_override : quarters * cus / 4, slots);
       if (most < tiles) continue;
-      int lo = (int)std::min<int64_t>(std::max<int64_t>(2, steps / most), shorter), hi = shorter; // blocks_at(hi) <= most
+      int lo = std::min(2, shorter), hi = shorter; // blocks_at(hi) <= most
       while (lo < hi) {
         const int mid = (lo + hi) / 2;
         if (blocks_at(mid) <= most)
@@ -324,10 +370,12 @@ void plan_prefill_splits(const mvr_paged_attention_args* a, const LiveSeqs& live
           lo = mid + 1;
       }
       shorter = lo;
-      if (lo >= longest) continue;
-      int part = 0;
-      const int64_t blocks = blocks_at(lo, &part);
-      const double cost = cost_us(blocks, part, 1.0) + merge_us((blocks + tiles - 1) / tiles) + 3;
+      if (lo >= most_steps) continue;
+      const Parts r = parts_at(lo);
+      // (In hand for several rounds, by what their estimates vary: 12% in F16, 4%
+      // in F32.)
+      const double cost = (cost_us(r.blocks, r.longest, r.busiest, 0.33 * r.longest) + merge_us(r.blocks) + 3) *
+                          (r.blocks <= cus ? 1.0 : a->dtype == MVR_DTYPE_F16 ? 1.12 : 1.04);
       if (cost < best || split_override > 1) {
         best = cost;
         part_steps = lo;

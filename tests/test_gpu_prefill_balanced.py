@@ -1,8 +1,8 @@
 """GPU parity of the prefill kernel's balanced grid: each row tile's keys in parts of about one length, a block per
 part, found from the device length tables, and a merge of the tiles that have several.
 
-The planner takes it for sequences of unequal lengths where a block per 128-row tile leaves CUs idle or waits for the
-longest.  Cases at the places where parts can go wrong: one and many parts per tile (over several rounds of the merge's
+The planner takes it for sequences of unequal lengths, and for (sequence, KV head) pairs that the 8 XCDs share
+unevenly, where a block per 128-row tile leaves CUs idle or waits for the longest.  Cases at the places where parts can go wrong: one and many parts per tile (over several rounds of the merge's
 8, and of the 4 that F32 keeps, up to 32), causal limits that leave a tile fewer key tiles than parts, more than 64
 sequences (the device scan's second round) with decodes among them, device tables that give more parts, or more tiles,
 than the host's did (the call then runs unsplit, its blocks striding over whole tiles), no workspace, token pages,
@@ -38,6 +38,7 @@ def _gpu():
 CASES = {
     "f32 3 ragged": ("f32", 28, 4, 128, 16, [117, 117, 117], [1860, 2320, 897], "tables", "balanced"),
     "f32 no workspace": ("f32", 28, 4, 128, 16, [117, 117, 117], [1860, 2320, 897], "no workspace", "unsplit"),
+    "f32 one length, 12 pairs": ("f32", 28, 4, 128, 16, [99] * 3, [700] * 3, "tables", "balanced"),
     "f32 other order": ("f32", 28, 4, 128, 16, [117, 30, 117], [1860, 2320, 97], "reversed", "balanced"),
     "f32 more parts": ("f32", 28, 4, 128, 16, [60, 60, 60], [3440, 3440, 2000], "one long", "more parts"),
     "f16 more parts": ("f16", 28, 4, 128, 16, [60, 60, 60], [3440, 3440, 2000], "one long", "more parts"),
@@ -51,7 +52,7 @@ CASES = {
     "f16 d64 token pages, past 8 parts": ("f16", 14, 2, 64, 24, [78, 18], [68, 4738], "tables", "balanced"),
     "f32 d64 4-token pages, past 8 parts": ("f32", 14, 2, 64, 4, [12, 37], [2102, 117], "tables", "balanced"),
     "f32 d64 causal": ("f32", 14, 2, 64, 16, [260, 118], [11, 1227], "tables", "balanced"),
-    "f16 d256, past 8 parts": ("f16", 8, 2, 256, 16, [44, 29], [136, 1777], "tables", "balanced"),
+    "f16 d256, past 8 parts": ("f16", 8, 2, 256, 16, [90, 17], [144, 2113], "tables", "balanced"),
     "f32 d96, past 8 parts": ("f32", 8, 2, 96, 16, [31, 101], [2335, 253], "tables", "balanced"),
     "f32 d160, past 4 parts": ("f32", 8, 2, 160, 16, [73, 27], [65, 1181], "tables", "balanced"),
     "f32 d192, past 4 parts": ("f32", 8, 2, 192, 16, [12, 134], [891, 74], "tables", "balanced"),

@@ -43,7 +43,7 @@ CASES = {
     "f16 12 pairs": ("f16", 28, 4, 128, 16, [50] * 3, [3000] * 3, "yes", 1),
     "f16 fresh": ("f16", 2, 1, 128, 16, [2000], [0], "yes", 1),
     "f16 near-fresh pair": ("f16", 2, 1, 128, 16, [1700] * 2, [3] * 2, "yes", 1),
-    "f16 other device tables": ("f16", 28, 4, 128, 16, [100, 37, 64], [40, 2100, 900], "equal", 1),
+    "f16 other device tables": ("f16", 32, 8, 128, 16, [100, 37, 64], [40, 2100, 900], "equal", 1),
     "f16 half the workspace": ("f16", 28, 4, 128, 16, [100], [4289], "yes", 0.5),
     "f16 no workspace": ("f16", 28, 4, 128, 16, [100], [4289], "yes", 0),
     "f16 chunks among decodes": ("f16", 32, 8, 128, 16, [1, 130, 1, 1, 130, 1], [90, 2000, 700, 5, 2000, 300], "yes", 1),
@@ -56,14 +56,14 @@ CASES = {
     "f32 d64 unequal, 4-token pages": ("f32", 14, 2, 64, 4, [41, 77], [1000, 3100], "yes", 1),
     "f16 d256 unequal": ("f16", 8, 2, 256, 16, [100, 33], [2500, 900], "yes", 1),
     "f32 d96 unequal": ("f32", 8, 2, 96, 16, [100, 33], [2500, 900], "yes", 1),
-    "f32 unequal, no tables": ("f32", 28, 4, 128, 16, [117] * 3, [1860, 2320, 897], "no", 1),
+    "f32 unequal, no tables": ("f32", 32, 8, 128, 16, [117] * 3, [1860, 2320, 897], "no", 1),
     "f16 d64": ("f16", 14, 2, 64, 16, [256], [2048], "yes", 1),
     "f16 d64 token pages": ("f16", 14, 2, 64, 24, [97] * 2, [3000] * 2, "yes", 1),
     "f16 d128 4-token pages": ("f16", 8, 2, 128, 4, [70], [3001], "yes", 1),
     "f16 d96": ("f16", 8, 2, 96, 16, [100], [3000], "yes", 1),
     "f16 d256": ("f16", 8, 2, 256, 16, [100], [3000], "yes", 1),
     "f32 one chunk": ("f32", 28, 4, 128, 16, [100], [4289], "yes", 1),
-    "f32 several rounds": ("f32", 28, 4, 128, 16, [99] * 3, [700] * 3, "yes", 1),
+    "f32 several rounds": ("f32", 32, 8, 128, 16, [99] * 3, [700] * 3, "yes", 1),
     "f32 d64": ("f32", 32, 8, 64, 16, [100], [3000], "yes", 1),
     "f32 d64 2-token pages": ("f32", 14, 2, 64, 4, [77], [1001], "yes", 1),
     "f32 d160": ("f32", 8, 2, 160, 16, [40], [1700], "yes", 1),

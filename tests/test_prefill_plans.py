@@ -115,3 +115,24 @@ def test_many_lengths(plan):
     seq = 300 + 130 * (np.arange(n) % 40) + 4000 * (np.arange(n) % 37 == 0)
     p = plan("f32", 4, 1, 128, 16, 30, int(seq.max()), True, [30] * n, seq)
     assert p["blocks"] > n, p
+
+
+# Row tiles near or past the CUs: dtype, heads, KV heads, head_dim, new tokens, cached tokens, grid.
+GRIDS = {
+    "f32 480 tiles": ("f32", 32, 8, 64, [627] * 3, [679, 428, 878], "unsplit"),
+    "f16 352 tiles": ("f16", 32, 8, 128, [700] * 2, [4888, 605], "unsplit"),
+    "f16 144 tiles": ("f16", 24, 8, 128, [119] * 6, [3543, 2990, 3425, 3645, 3113, 1695], "unsplit"),
+    "f16 one sequence, 56 tiles": ("f16", 28, 4, 128, [256], [2048], "parts"),
+    "f32 160 tiles of one length": ("f32", 32, 8, 128, [151] * 4, [1593] * 4, "parts"),
+    "f32 12 pairs of one length": ("f32", 28, 4, 128, [151] * 3, [1593] * 3, "balanced"),
+}
+
+
+@pytest.mark.parametrize("name", list(GRIDS))
+def test_grids_of_many_tiles(plan, name):
+    """More blocks than CUs run in rounds, each as long as a part: only where that is shorter is a call split."""
+    dtype, hq, hkv, d, q, cached, grid = GRIDS[name]
+    seq = np.array(cached) + q
+    p = plan(dtype, hq, hkv, d, 16, max(q), int(seq.max()), True, q, seq)
+    assert p["prefill"]
+    assert ("balanced" if p["blocks"] else "parts" if p["kv_splits"] > 1 else "unsplit") == grid, p
