@@ -30,9 +30,9 @@
 // Blocks of one (sequence, KV head) are mapped onto one XCD (workgroups are
 // dispatched round-robin over the 8 XCDs), so their shared K/V stays in that
 // XCD's L2.  Grids that leave CUs idle split each tile's keys into as many
-// parts (kv_splits), and grids of unequal tiles run balanced, in parts of about
-// one length: a block per part, combined by prefill_merge_kernel from an fp32
-// partial workspace.
+// parts (kv_splits), and grids of unequal tiles, or of pairs that the XCDs share
+// unevenly, run balanced, in parts of about one length: a block per part,
+// combined by prefill_merge_kernel from an fp32 partial workspace.
 #include "paged_prefill.hpp"
 #include "wave_scan.hpp"
 
